@@ -69,8 +69,9 @@ __global__ __launch_bounds__(THREADS) void k_cull_views(CullLaunch a) {
     return fabsf(c0) < tol && fabsf(c1) < tol && fabsf(c2 - 0.5f) < 0.5f;
   };
 
+  if (persistent_idle(num_tiles)) return;
   while (true) {
-    if (tid == 0) s_tile = atomicAdd(&a.counters[kCtrCull], 1u);
+    if (tid == 0) s_tile = take_ticket(&a.counters[kCtrCull], num_tiles);
     __syncthreads();
     const uint32_t t = s_tile;
     if (t >= num_tiles) break;
@@ -151,7 +152,6 @@ __global__ __launch_bounds__(THREADS) void k_cull_views(CullLaunch a) {
     }
     __syncthreads();
   }
-  finish_persistent(&a.counters[kCtrCull], &a.counters[kDone + kCtrCull]);
 }
 
 // Onesweep upsweep: the digit histograms of every radix pass over a view's

@@ -371,10 +371,11 @@ __global__ __launch_bounds__(THREADS) void k_bin(BinLaunch a) {
     counters[kPairs] = 0u;
     counters[kPairOverflow] = 0u;
   }
+  if (persistent_idle(num_tiles)) return;
   const uint32_t tiles_x = a.uniforms[v].tiles_x;
 
   while (true) {
-    if (tid == 0) s_tile = atomicAdd(&counters[kCtrBin], 1u);
+    if (tid == 0) s_tile = take_ticket(&counters[kCtrBin], num_tiles);
     __syncthreads();
     const uint32_t t = s_tile;
     if (t >= num_tiles) break;
@@ -509,7 +510,6 @@ __global__ __launch_bounds__(THREADS) void k_bin(BinLaunch a) {
   }
   for (int i = tid; i < a.pair_passes * 256; i += THREADS)
     if (s_hist[i]) atomicAdd(&a.hist[v * a.hist_stride + i], s_hist[i]);
-  finish_persistent(&counters[kCtrBin], &counters[kDone + kCtrBin]);
 }
 
 // Run boundaries of the tile-sorted pair keys, four keys per thread.

@@ -64,6 +64,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
   uint32_t n = counters[a.count_slot];
   if (n > a.count_cap) n = a.count_cap;
   const uint32_t num_tiles = (n + TILE - 1) / TILE;
+  if (persistent_idle(num_tiles)) return;
   const int shift = a.shift;
 
   {  // global exclusive digit starts
@@ -249,7 +250,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
   };
 
   while (true) {
-    if (tid == 0) s_tile = atomicAdd(tile_counter, 1u);
+    if (tid == 0) s_tile = take_ticket(tile_counter, num_tiles);
     for (int i = tid; i < WAVES * RADIX; i += THREADS) s_wave_hist[i] = 0u;
     __syncthreads();
     const uint32_t t = s_tile;
@@ -258,7 +259,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     if (left >= (uint32_t)TILE) tile_pass(Flag<true>{}, t, (uint32_t)TILE);
     else tile_pass(Flag<false>{}, t, left);
   }
-  finish_persistent(tile_counter, counters + kDone + a.tile_slot);
 }
 
 template <int BITS>

@@ -39,7 +39,6 @@ enum CounterSlot : int {
   kCtrBin = 5,
   kCtrPair0 = 6,    // .. kCtrPair0 + 2
   kCtrCount = 9,
-  kDone = 16,       // done counters mirror tile counters at +16
   kVisible = 32,
   kPairs = 33,
   kPairOverflow = 34,
