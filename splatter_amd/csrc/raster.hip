@@ -675,10 +675,9 @@ __global__ __launch_bounds__(256, MODE == 3 ? (B == 128 ? (F32 ? 6 : 7) : 5) : 1
   // Block -> (view, tile).  First the heavy tiles of every view (their
   // count rounded up to 8 blocks; with split_heavy, mode 3 only, four blocks
   // per heavy tile, one per 8x8 quadrant, each wave two of its rows), then
-  // each view's other tiles in a slot range of slots_per_view blocks,
-  // banded per XCD: blocks are dealt round-robin to the 8 XCDs, and each
-  // XCD takes a contiguous run of rows (neighbouring tiles share records in
-  // its L2).  A heavy tile's pixels wait on their own long chains of
+  // each view's other tiles in a slot range of slots_per_view blocks: blocks
+  // are dealt round-robin to the 8 XCDs, and the XCDs take runs of kXcdRun
+  // neighbouring tiles in turn (kXcdRun has why).  A heavy tile's pixels wait on their own long chains of
   // blends; with one view on the device the other blocks are soon done, and
   // sixteen waves on a tile instead of four shorten its chains' wave-wide
   // steps (each step waits for the busiest of 16 pixels, not 64).
@@ -712,8 +711,8 @@ __global__ __launch_bounds__(256, MODE == 3 ? (B == 128 ? (F32 ? 6 : 7) : 5) : 1
       b -= heavy_blocks;
       v = b / a.slots_per_view;
       if (v >= nv) return;
-      const uint32_t k = b % a.slots_per_view, per = a.slots_per_view / 8;
-      const uint32_t p = (k & 7u) * per + (k >> 3);
+      const uint32_t k = b % a.slots_per_view;
+      const uint32_t p = ((k >> 3) / kXcdRun * 8u + (k & 7u)) * kXcdRun + (k >> 3) % kXcdRun;
       const uint32_t h = a.longest_first ? a.counters[(size_t)v * kCounterWords + kHeavyTiles] : 0u;
       const uint32_t tv = a.uniforms[v].tiles_x * a.uniforms[v].tiles_y;
       if (p >= tv - h) return;

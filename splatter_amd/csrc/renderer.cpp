@@ -471,7 +471,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.views = (int)nv;
     launch_ranges(a, q);
   }
-  const uint32_t slots = ((b.max_tiles + 7) / 8) * 8;
+  const uint32_t slots = div_up(b.max_tiles, 8 * kXcdRun) * 8 * kXcdRun;
   const uint32_t heavy_cap = std::max<uint32_t>(8, slots / 8);
   // A single view rasters in 256-entry batches, its longest tiles first:
   // with only one view's tiles on the device the longest ones set the

@@ -27,6 +27,13 @@ struct Uniforms {
 };
 
 constexpr int kTileSize = 16;        // raster tile edge in pixels (16x16 = 256 lanes)
+// Neighbouring screen tiles that the raster gives to one XCD before the next
+// XCD's run.  Short, because views are uneven: with an eighth of the screen to
+// each XCD, the one with the horizon was still at work when the ones with the
+// sky were done (16 views of 6M splats: a pass of 12.84 ms so, 11.50 with
+// runs of 4, 11.65 with 16, 11.48 with 120; one 4K view 1.57, 1.48, 1.45 and
+// 1.47 ms; one 1080p view of 1M 561, 550, 562 and 565 us).
+constexpr uint32_t kXcdRun = 4;
 constexpr int kMaxDepthPasses = 4;   // 30-bit depth keys: 4 x 8 bits or 3 x 10 bits
 constexpr int kMaxPairPasses = 3;    // screen-tile ids up to 24 bits
 constexpr int kRecordFloat4 = 3;     // 48-byte record: rgba | A00 A10 A01 A11 | tx ty box box
@@ -177,7 +184,7 @@ struct OrderLaunch {
 
 struct RasterLaunch {
   const uint32_t* order; size_t order_stride;
-  uint32_t slots_per_view;   // multiple of 8, >= the largest view's tile count
+  uint32_t slots_per_view;   // multiple of 8 * kXcdRun, >= the largest view's tile count
   uint32_t heavy_cap;
   const uint32_t* pair_vals; size_t pair_stride;
   const float4* records; size_t rec_stride;
