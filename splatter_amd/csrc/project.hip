@@ -239,6 +239,10 @@ __device__ void pixel_box(float A00, float A10, float A01, float A11, float tx, 
 // pairs as LDS allows: every lane projects one pair, lanes do not idle on
 // views that do not see their splat even when a frame has one view, and the
 // lanes of one splat read its attributes from the same cache lines.
+// Small scenes have fewer cull tiles than the chip has places for blocks, and
+// a tile's sixteen groups run one after another: `parts` blocks then share a
+// tile, each with its own run of groups (every one of them still counts the
+// tile's masks, 4096 words, for the entries before its own).
 template <int L>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_project(ProjectLaunch a) {
   constexpr int THREADS = kCullThreads, ITEMS = kCullItems, WAVES = THREADS / kWave, TILE = kCullTile;
@@ -421,7 +425,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     }
   };
 
-  for (uint32_t t = blockIdx.x; t < num_tiles; t += gridDim.x) {
+  for (uint32_t part = blockIdx.x; part < num_tiles * a.parts; part += gridDim.x) {
+    const uint32_t t = part / a.parts;
+    const int groups = ITEMS / (int)a.parts, j0 = (int)(part % a.parts) * groups;
     // per view: exclusive offsets of the (item, wave) groups inside the tile.
     // The sixteen masks are requested before any is used (past the end a
     // lane reads splat 0's and drops it), so the loads do not wait in turn.
@@ -471,11 +477,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
       __syncthreads();
       uint32_t listed = 0;  // pairs in the list (uniform across the block)
       // each group's masks are requested one group ahead
-      uint32_t ahead = a.vis[t * TILE + tid < n ? t * TILE + tid : 0u];
-      for (int j = 0; j < ITEMS; ++j) {
+      const uint32_t first = t * TILE + j0 * THREADS + tid;
+      uint32_t ahead = a.vis[first < n ? first : 0u];
+      for (int j = j0; j < j0 + groups; ++j) {
         const uint32_t base = j * THREADS;
         const uint32_t all = t * TILE + base + tid < n ? ahead : 0u;
-        if (j + 1 < ITEMS) {
+        if (j + 1 < j0 + groups) {
           const uint32_t nx = t * TILE + base + THREADS + tid;
           ahead = a.vis[nx < n ? nx : 0u];
         }

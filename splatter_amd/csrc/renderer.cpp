@@ -340,7 +340,15 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_words = cull_used;
       a.clear_a_stride = r->cull_tiles;
     }
-    a.grid = clampg(div_up(n, kCullTile), cus * 3);  // three resident blocks per CU
+    // Three resident blocks per CU, each tile on as many blocks as fill one
+    // round of them: 1M splats (245 tiles) on 490 blocks 42 us, on 245 59;
+    // 20k (5 tiles) on 80 blocks 12 us, on 5 about 55; 5 views of 300k
+    // (74 tiles) on 592 blocks 46 us, on 74 140.  Two or four rounds of finer
+    // parts were no faster (1M 43 and 47 us, 1.5M 69 and 75 against 65 us).
+    const uint64_t tiles = div_up(n, kCullTile);
+    a.parts = 1;
+    while (a.parts < (uint32_t)kCullItems && tiles * a.parts * 2 <= (uint64_t)cus * 3) a.parts *= 2;
+    a.grid = clampg(tiles * a.parts, cus * 3);
     launch_project(a, qq);
   };
   mark(1);

@@ -131,6 +131,7 @@ struct ProjectLaunch {
   const Uniforms* uniforms;
   const uint32_t* vis;
   const uint32_t* tile_prefix; size_t tp_stride;
+  uint32_t parts;                           // blocks that share a cull tile: 1, 2, 4, 8 or 16
   int sh_order;
   int use_covariance_for_scale;
   int use_unaligned_rectangles;

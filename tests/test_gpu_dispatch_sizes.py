@@ -27,3 +27,36 @@ def test_every_tile_is_drawn_once(width, height):
     other = sa.Frame(device(), 40, 40)  # the same view beside a smaller one, whose tiles end inside a turn
     case.renderer.render_views([other, case.frame], [case.cam] * 2, [case.view] * 2, case.scene)
     assert np.array_equal(case.frame.read()[..., [2, 1, 0, 3]], img)
+
+
+# 48, 96, 192 and 384 cull tiles of 4096 splats are the most that 16, 8, 4 and
+# 2 blocks share on 256 CUs; one splat more starts the next form, with a last
+# tile of one splat
+@pytest.mark.parametrize("count", [1, 255, 4097, 48 * 4096, 48 * 4096 + 1, 96 * 4096 + 1, 192 * 4096 + 1,
+                                   384 * 4096 + 1])
+@pytest.mark.parametrize("views", [1, 3])
+def test_blocks_that_share_a_cull_tile(count, views):
+    say(f"{count} splats, {views} views")
+    w = Workload("gaussian", count, seed=33)
+    cfg = config(max_splat_count=count, max_views=views, tile_pairs_per_splat=8)
+    r = sa.Renderer(device(), cfg)
+    scene = sa.Scene(r, count)
+    records = w.all()
+    scene.load_records(0, records)
+    splats = ob.decode(records)
+    poses = [sphere_pose(40 + v, radius=4) for v in range(views)]
+    frames = [sa.Frame(device(), 96, 64) for _ in range(views)]
+    r.render_views(frames, [p[0] for p in poses], [p[1] for p in poses], scene)
+    for v, (cam, view) in enumerate(poses):
+        r.select_view(v)
+        _, idx = r.read_entries()
+        u = ob.uniforms(cam, view, 96, 64)
+        _, oidx = ob.cpu_depth_sort(splats["center"], ob.vp_of(u), 1.1)
+        assert np.array_equal(idx, oidx)
+        if not len(idx):
+            continue
+        sub = np.unique(np.linspace(0, len(idx) - 1, min(len(idx), 3000)).astype(np.int64))
+        rec = r.read_records()[sub]
+        orec, _ = ob.project(splats[idx[sub]], u, cfg.spherical_harmonics_order, cfg.use_covariance_for_scale)
+        assert np.array_equal(rec[:, :4], orec[:, :4])
+        assert normwise_rel(rec[:, 4:], orec[:, 4:]).max() <= RECORD_TOL
