@@ -286,12 +286,26 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   const uint32_t per_view = std::max<uint32_t>(1, cus * 4 / nv);
   // radix-sort tiles: one 1024-lane, two 512-lane or four 256-lane blocks per CU, shared
   // by the views (which sort side by side, so their look-back chains overlap)
-  // A single view sorts in 16384-key tiles whatever the batches use: with
-  // one view on the device the look-back chains set the sort's time, and
-  // larger tiles shorten them (the autotuner picks the batches' tile).
-  const int sort_threads = nv == 1 ? kSortThreadsXL : r->sort_threads;
-  const uint32_t sort_tile = (uint32_t)sort_threads * kSortItems;
-  const uint32_t sort_per_view = std::max<uint32_t>(1, cus * 4 * kSortThreads / sort_threads / nv);
+  // A single view picks its tile by the scene's size, whatever the batches
+  // use (the autotuner picks the batches' tile).  Small scenes leave CUs idle
+  // and pay for a tile's own chain (a 1024-lane block ranks four waves a
+  // SIMD), large ones for the look-back over many tiles; us, one view on
+  // MI355X, depth sort / pair sort in tiles of 4096, 8192 and 16384 keys:
+  //   20k splats   54 / 16    58 / 17    72 / 22
+  //   100k         53 / 33    59 / 32    75 / 38
+  //   1M           67 / 43    67 / 40    79 / 43
+  //   1.5M         72 / 44    69 / 40    79 / 44
+  //   3M at 4K     93 / 98    84 / 83    91 / 79
+  //   6M          126 / 105  103 / 85   101 / 85
+  const auto one_view = [n](uint64_t narrow, uint64_t wide) {
+    return n <= narrow ? kSortThreads : n <= wide ? kSortThreadsWide : kSortThreadsXL;
+  };
+  const int depth_threads = nv == 1 ? one_view(1u << 19, 1u << 22) : r->sort_threads;
+  const int pair_threads = nv == 1 ? one_view(1u << 18, 1u << 21) : r->sort_threads;
+  const auto sort_grid = [&](uint64_t keys, int threads) {
+    const uint32_t per_view = std::max<uint32_t>(1, cus * 4 * kSortThreads / threads / nv);
+    return (int)std::max<uint64_t>(1, std::min<uint64_t>(div_up(keys, (uint64_t)threads * kSortItems), per_view));
+  };
   const size_t cap = r->cap;
   const size_t sort_stride = r->sort_words * kMaxDepthPasses;
   const size_t pair_stride_status = r->pair_words * kMaxPairPasses;
@@ -390,8 +404,8 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_words = sort_used;
       a.clear_a_stride = sort_stride;
     }
-    a.threads = sort_threads;
-    a.grid_x = clampg(div_up(n, sort_tile), sort_per_view);
+    a.threads = depth_threads;
+    a.grid_x = sort_grid(n, depth_threads);
     a.views = (int)nv;
     // keys are below 2^30 (0 < clip.z < 1): the last 8-bit pass needs 6 bits
     launch_sort_pass(std::min(bits, 30 - p * bits), a, q);
@@ -454,8 +468,8 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_words = r->pair_words;
       a.clear_a_stride = pair_stride_status;
     }
-    a.threads = sort_threads;
-    a.grid_x = clampg(div_up(r->pair_cap, sort_tile), sort_per_view);
+    a.threads = pair_threads;
+    a.grid_x = sort_grid(r->pair_cap, pair_threads);
     a.views = (int)nv;
     // tile keys are below max_tiles: the last pass takes only their top bits
     launch_sort_pass(std::max(5, std::min(8, tile_bits - 8 * p)), a, q);

@@ -60,3 +60,31 @@ def test_blocks_that_share_a_cull_tile(count, views):
         orec, _ = ob.project(splats[idx[sub]], u, cfg.spherical_harmonics_order, cfg.use_covariance_for_scale)
         assert np.array_equal(rec[:, :4], orec[:, :4])
         assert normwise_rel(rec[:, 4:], orec[:, 4:]).max() <= RECORD_TOL
+
+
+# one view sorts depths in 4096-key tiles up to 2^19 splats, in 8192-key tiles
+# up to 2^22 and in 16384-key tiles beyond; pairs change at 2^18 and 2^21
+@pytest.mark.parametrize("count", [1 << 18, (1 << 18) + 1, 1 << 19, (1 << 19) + 1, (1 << 21) + 1, (1 << 22) + 1])
+@pytest.mark.parametrize("bits", [8, 10])
+def test_sort_tile_of_one_view(count, bits):
+    say(f"{count} splats, {bits}-bit digits")
+    r = sa.Renderer(device(), config(max_splat_count=count, radix_bits_per_digit=bits, tile_pairs_per_splat=8,
+                                     max_views=2))
+    w = Workload("gaussian", count, seed=35)
+    scene = sa.Scene(r, count)
+    centers = np.empty((count, 3), np.float32)
+    for first, rec in w.chunks():
+        scene.load_records(first, rec)
+        centers[first:first + len(rec)] = rec["center"]
+    cam, view = sphere_pose(35, radius=5)
+    frames = [sa.Frame(device(), 640, 360) for _ in range(2)]
+    r.render_frame(frames[0], cam, view, scene)
+    keys, idx = r.read_entries()
+    okeys, oidx = ob.cpu_depth_sort(centers, ob.vp_of(ob.uniforms(cam, view, 640, 360)), 1.1)
+    assert np.array_equal(idx, oidx) and np.array_equal(keys, okeys)
+    # a batch sorts its pairs in the configured tile: the same lists, the same image
+    r.render_views(frames[::-1], [cam] * 2, [view] * 2, scene)
+    assert np.array_equal(frames[0].read(), frames[1].read())
+    batch = frames[0].read()
+    r.render_frame(frames[0], cam, view, scene)
+    assert np.array_equal(frames[0].read(), batch)
