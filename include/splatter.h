@@ -99,13 +99,13 @@ typedef struct spl_configuration {
                                              sub-blocks side by side;
                                              3 (default): for 32 list slots at a time each lane finds
                                              the entries that can cover its pixel (per row, from the
-                                             rectangles' column intervals), then walks them on its own;
-                                             one view also splits its heaviest tiles over four blocks
-                                             (all the same image) */
+                                             rectangles' column intervals), then walks them on its own
+                                             (all the same image; tiles with the longest lists have a
+                                             walk of their own in every mode) */
     uint32_t raster_batch;                /* entries a raster block stages per batch: 128 or 256
-                                             (batches of two or more views; one view uses 256) */
-    uint32_t raster_longest_first;        /* 1: tiles with the longest lists start first (same image;
-                                             batches of two or more views; one view always does) */
+                                             (batches of two or more views; one view uses 128) */
+    uint32_t raster_longest_first;        /* 0 or 1, no effect: tiles with the longest lists always
+                                             start first */
 } spl_configuration;
 
 const char* spl_last_error(void);

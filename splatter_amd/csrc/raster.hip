@@ -8,191 +8,20 @@
 //          the digit histograms of the tile ids for the stable pair sort.
 //  ranges  [start, end) of each tile's run in the tile-sorted pair list.
 //  raster  one 256-lane block per tile, one lane per pixel, one wave per 8x8
-//          quadrant (one view: the heaviest tiles on four blocks, one per
-//          quadrant, two rows a wave): records staged in LDS 128 or 256 at a
-//          time, each wave keeping the ones that can reach its
-//          still-transparent pixels, blended front to back in draw order with
-//          the reference's blend state (colour = src*DstAlpha + dst, alpha =
-//          dst*(1-srcA), cleared to (0,0,0,1)), the unorm8 target emulated by
-//          clamping the source and re-quantising after every blend; a wave
-//          stops once its pixels' transmittance is 0, a tile once all four
-//          have.
-#include "spl_device.h"
-#include "spl_internal.h"
+//          quadrant: records staged in LDS 128 or 256 at a time, each wave
+//          keeping the ones that can reach its still-transparent pixels,
+//          blended front to back in draw order with the reference's blend
+//          state (colour = src*DstAlpha + dst, alpha = dst*(1-srcA), cleared
+//          to (0,0,0,1)), the unorm8 target emulated by clamping the source
+//          and re-quantising after every blend; a wave stops once its pixels'
+//          transmittance is 0, a tile once all four have.  The tiles with the
+//          longest lists get blocks of their own (raster_heavy.h).
+#include "raster_common.h"
+#include "raster_heavy.h"
 
 namespace spl {
 
 namespace {
-
-// The fragment's Gaussian e^(-|tc|^2 / 2) (shaders.wgsl:586) is evaluated as
-// 2^-(|S tc|^2) with S = sqrt(log2(e) / 2) folded into each entry's inverse
-// map, so a pixel costs two fused products per coordinate and one exp2.
-constexpr float kGaussScale = 0.84932180f;
-
-// 2^y for y <= 0: y = k + f with k = rint(y), |f| <= 1/2, a degree-5
-// relative minimax polynomial of 2^f (constant term 1, so exact at
-// integers; within 3 ulp of exp2) in fused Horner form, then ldexp by k
-// (exact while the result stays normal).  Only correctly rounded IEEE
-// operations (fma, rint, ldexp), so it rounds the same on the CPU and the
-// GPU.  The oracle clamps y at -125 first; below -8 every alpha is under the
-// 1/255 fragment threshold either way, so the pixels agree without it.
-__device__ __forceinline__ float spl_exp2(float y) {
-  const float k = rintf(y);
-  const float f = y - k;
-  float p = 1.32764713e-3f;
-  p = fmaf(p, f, 9.67554189e-3f);
-  p = fmaf(p, f, 5.55071309e-2f);
-  p = fmaf(p, f, 2.40221202e-1f);
-  p = fmaf(p, f, 6.93146944e-1f);
-  p = fmaf(p, f, 1.0f);
-  return ldexpf(p, (int)k);
-}
-
-__device__ __forceinline__ float q8(float x) {
-  x = fminf(fmaxf(x, 0.0f), 1.0f);
-  return floorf(x * 255.0f + 0.5f);
-}
-
-__device__ __forceinline__ float clamp01(float x) { return fminf(fmaxf(x, 0.0f), 1.0f); }
-
-// Pixel centres in the view plane are q = (sx px + ox, sy py + oy)
-// (shaders.wgsl:561 inverted).  Each staged entry folds this map into its
-// own: with e = o - t the coverage coordinate is affine in the integer
-// pixel coordinates,
-//   unaligned:     u = au px + bu py + cu,  w = av px + bv py + cv
-//   axis-aligned:  dx = sx px + ex,  dy = sy py + ey  (then u, w from dx, dy)
-// so a pixel costs two fused products per coordinate.
-struct PixelMap {
-  float sx, ox, sy, oy;
-};
-
-__device__ __forceinline__ PixelMap pixel_map(const Uniforms& u) {
-  const float Wf = (float)u.image_size[0], Hf = (float)u.image_size[1], vw = u.view_size[0], vh = u.view_size[1];
-  PixelMap p;
-  p.sx = (2.0f * vw) / Wf;
-  p.ox = vw / Wf - vw;
-  p.sy = -(2.0f * vh) / Hf;
-  p.oy = vh - vh / Hf;
-  return p;
-}
-
-// The staged form of a record (g0: colour and opacity, g1: the rectangle's
-// axes, g2: its centre and pixel box): e0 the inverse map scaled by S (and,
-// unaligned, folded with the pixel map), e1 its translation, the coverage
-// half-extent and the opacity, e2 the colour.
-template <bool UNALIGNED>
-__device__ __forceinline__ void prepare_entry(const float4& g0, const float4& g1, const float4& g2, const PixelMap& pm,
-                                              float margin, float4& e0, float4& e1, float4& e2) {
-  const float A00 = g1.x, A10 = g1.y, A01 = g1.z, A11 = g1.w;
-  const float det = A00 * A11 - A10 * A01;
-  const float rs = (1.0f / det) * kGaussScale;  // inverse map scaled by S
-  const float i00 = A11 * rs, i01 = -A01 * rs, i10 = -A10 * rs, i11 = A00 * rs;
-  const float ex = pm.ox - g2.x, ey = pm.oy - g2.y;
-  // unaligned: the rectangle |tc| < margin in scaled coordinates;
-  // axis-aligned: a square of half-side radius * margin in the view plane
-  const float half = UNALIGNED ? margin * kGaussScale
-                               : sqrtf(fmaxf(A00 * A00 + A10 * A10, A01 * A01 + A11 * A11)) * margin;
-  if constexpr (UNALIGNED) {
-    e0 = make_float4(i00 * pm.sx, i01 * pm.sy, i10 * pm.sx, i11 * pm.sy);
-    e1 = make_float4(fmaf(i00, ex, i01 * ey), fmaf(i10, ex, i11 * ey), half, g0.w);
-  } else {
-    e0 = make_float4(i00, i01, i10, i11);
-    e1 = make_float4(ex, ey, half, g0.w);
-  }
-  e2 = make_float4(g0.x, g0.y, g0.z, 0.0f);
-}
-
-// Can entry (m, t) cover a pixel centre of the pixel box [x0, x1] x
-// [y0, y1]?  The tested coordinates are affine in the pixel, so their exact
-// range over the box sits at the corners; the slack (relative to the
-// magnitudes the per-pixel evaluation adds up) is far above its rounding.
-template <bool UNALIGNED>
-__device__ __forceinline__ bool range_meets(const float4& m, const float4& t, float x0, float x1, float y0, float y1,
-                                            const PixelMap& pm) {
-  const float h = t.z;
-  float a0, a1, b0, b1, sa, sb;  // ranges of the tested coordinates, and slack
-  if constexpr (UNALIGNED) {
-    a0 = (fminf(m.x * x0, m.x * x1) + fminf(m.y * y0, m.y * y1)) + t.x;
-    a1 = (fmaxf(m.x * x0, m.x * x1) + fmaxf(m.y * y0, m.y * y1)) + t.x;
-    b0 = (fminf(m.z * x0, m.z * x1) + fminf(m.w * y0, m.w * y1)) + t.y;
-    b1 = (fmaxf(m.z * x0, m.z * x1) + fmaxf(m.w * y0, m.w * y1)) + t.y;
-    sa = 1e-4f * (((fabsf(m.x) * x1 + fabsf(m.y) * y1) + fabsf(t.x)) + h);
-    sb = 1e-4f * (((fabsf(m.z) * x1 + fabsf(m.w) * y1) + fabsf(t.y)) + h);
-  } else {
-    a0 = fmaf(pm.sx, x0, t.x); a1 = fmaf(pm.sx, x1, t.x);  // sx > 0
-    b0 = fmaf(pm.sy, y1, t.y); b1 = fmaf(pm.sy, y0, t.y);  // sy < 0
-    sa = 1e-4f * ((pm.sx * x1 + fabsf(t.x)) + h);
-    sb = 1e-4f * ((fabsf(pm.sy) * y1 + fabsf(t.y)) + h);
-  }
-  return a1 + sa >= -h && a0 - sa < h && b1 + sb >= -h && b0 - sb < h;
-}
-
-// Coverage of the pixel centre (pxf, pyf) by entry (m, t): the scaled
-// texture coordinate (u, w2) and whether it lies in the rectangle.
-template <bool UNALIGNED>
-__device__ __forceinline__ bool covers(const float4& m, const float4& t, float pxf, float pyf, const PixelMap& pm,
-                                       float& u, float& w2) {
-  const float h = t.z;
-  if constexpr (UNALIGNED) {
-    u = fmaf(m.x, pxf, fmaf(m.y, pyf, t.x));  // S * texture coordinate
-    w2 = fmaf(m.z, pxf, fmaf(m.w, pyf, t.y));
-    return fmaxf(fabsf(u), fabsf(w2)) < h;
-  } else {
-    const float dx = fmaf(pm.sx, pxf, t.x), dy = fmaf(pm.sy, pyf, t.y);
-    u = fmaf(m.x, dx, m.y * dy);
-    w2 = fmaf(m.z, dx, m.w * dy);
-    return fmaxf(fabsf(dx), fabsf(dy)) < h;
-  }
-}
-
-// One pixel's blend state: colour and transmittance, unorm8 codes or f32.
-template <bool F32>
-struct PixelState {
-  float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f, tr = F32 ? 1.0f : 255.0f;
-
-  // One fragment: alpha (shaders.wgsl:585-589) and the blend.  in: the
-  // coverage test's verdict, for walks over candidates that did not pass
-  // it yet; an uncovered fragment blends nothing.
-  __device__ __forceinline__ void shade(float u, float w2, float opacity, const float4& col, bool in) {
-    float alpha = opacity * spl_exp2(-fmaf(u, u, w2 * w2));
-    if constexpr (!F32) {
-      // unorm8 codes C, T: rint(s * T + C) (s clamped, sum capped at
-      // 255) and rint(T * (1 - a)): the ideal 8-bit blender.  Below the
-      // threshold alpha becomes 0, which leaves C and T as they are
-      // (they hold integers; clamp01 of a NaN product is 0), so no
-      // branch is needed.
-      alpha = in && alpha >= 1.0f / 255.0f ? alpha : 0.0f;
-      const float sr = col.x * alpha, sg = col.y * alpha, sb = col.z * alpha;
-      // the source alpha needs no clamp: the opacity is a sigmoid (or 1
-      // in the dev-test scene) and spl_exp2 of a non-positive argument is
-      // at most 1 (p(f) <= p(0) = 1 when rint(y) = 0, p(f) / 2 < 1 below),
-      // so alpha is in [0, 1] after the threshold
-      const float sa = alpha;
-      c0 = fminf(rintf(fmaf(clamp01(sr), tr, c0)), 255.0f);
-      c1 = fminf(rintf(fmaf(clamp01(sg), tr, c1)), 255.0f);
-      c2 = fminf(rintf(fmaf(clamp01(sb), tr, c2)), 255.0f);
-      tr = rintf(fmaf(-sa, tr, tr));
-    } else if (in && alpha >= 1.0f / 255.0f) {
-      const float sr = col.x * alpha, sg = col.y * alpha, sb = col.z * alpha;
-      const float da = tr;
-      c0 = fmaf(sr, da, c0);
-      c1 = fmaf(sg, da, c1);
-      c2 = fmaf(sb, da, c2);
-      tr = fmaf(-alpha, da, da);
-    }
-  }
-
-  // The pixel's final value, as the frame stores it.
-  __device__ __forceinline__ uint32_t packed(bool bgra) const {
-    uint32_t r, g, b, al;
-    if (!F32) {
-      r = (uint32_t)c0; g = (uint32_t)c1; b = (uint32_t)c2; al = (uint32_t)tr;
-    } else {
-      r = (uint32_t)q8(c0); g = (uint32_t)q8(c1); b = (uint32_t)q8(c2); al = (uint32_t)q8(tr);
-    }
-    return bgra ? (b | (g << 8) | (r << 16) | (al << 24)) : (r | (g << 8) | (b << 16) | (al << 24));
-  }
-};
 
 // Per-lane walk over one run of cnt <= 32 entries (cm, ct, cc: their three
 // staged rows, in list order, in LDS) of a wave's 8x8 region with top-left
@@ -517,6 +346,7 @@ __global__ __launch_bounds__(256) void k_tile_ranges(RangesLaunch a) {
   const uint32_t v = blockIdx.y;
   if (a.clear_a) clear_words(a.clear_a + v * a.clear_a_stride, a.clear_a_words);
   if (a.clear_b) clear_words(a.clear_b + v * a.clear_b_stride, a.clear_b_words);
+  if (blockIdx.x == 0 && v == 0 && threadIdx.x <= kHeavyClasses) a.counters[kHeavyAll + threadIdx.x] = 0u;
   const uint32_t* keys = a.pair_keys + v * a.pair_stride;  // 16-byte aligned: pair_stride % 4 == 0
   uint2* ranges = a.ranges + v * a.ranges_stride;
   const uint32_t tiles = a.uniforms[v].tiles_x * a.uniforms[v].tiles_y;
@@ -548,100 +378,37 @@ __global__ __launch_bounds__(256) void k_tile_ranges(RangesLaunch a) {
   }
 }
 
-// Raster order of a view's tiles: the tiles with the longest pair lists
-// ("heavy": at least heavy_mult x the mean and heavy_min pairs, at most
-// heavy_cap of them, whole log2 classes only) first, longest class first,
-// then every other tile in row-major order.  A heavy tile blends thousands
-// of entries per pixel, one after another; started last, it would outlast
-// the rest of the frame.  The heavy tiles in classes of at least
-// split_mult x the mean (and 2048 pairs) are counted apart: the raster may
-// give each of them four blocks.
-__global__ __launch_bounds__(1024) void k_tile_order(OrderLaunch a) {
-  constexpr int THREADS = 1024;
-  __shared__ uint32_t s_cnt[32];
-  __shared__ uint32_t s_cur[32];
-  __shared__ uint32_t s_tmp[THREADS / kWave];
-  __shared__ uint32_t s_cut;
-  const uint32_t v = blockIdx.y, tid = threadIdx.x;
+// The tiles whose lists are long enough to set the raster's time by
+// themselves ("heavy", kHeavyShare has the rule).  k_raster gives each eight
+// blocks, longest first: they are listed by length in kHeavyClasses lists (the
+// last for 16 x the threshold and more), and the top bit of a listed tile's
+// range start tells its ordinary block to leave it alone.  One thread per
+// tile; appends are atomics on counters that k_tile_ranges zeroed.  (The one
+// block that put the tiles in order before took 14 us at 1080p and 65 at 4K;
+// this takes 4 to 8.)
+__global__ __launch_bounds__(256) void k_heavy_tiles(HeavyLaunch a) {
+  const uint32_t v = blockIdx.y, t = blockIdx.x * 256 + threadIdx.x;
   const uint32_t T = a.uniforms[v].tiles_x * a.uniforms[v].tiles_y;
-  const uint2* ranges = a.ranges + v * a.ranges_stride;
-  uint32_t* order = a.order + v * a.order_stride;
-  uint32_t* counters = a.counters + (size_t)v * kCounterWords;
-  uint32_t k = counters[kPairs];
-  if (k > a.pair_cap) k = a.pair_cap;
-  const uint32_t mean = T ? k / T : 0u;
-  const uint32_t thr = max(a.heavy_mult * mean, a.heavy_min);
-  if (tid < 32) s_cnt[tid] = 0u;
-  __syncthreads();
-  const uint32_t chunk = (T + THREADS - 1) / THREADS;
-  const uint32_t t0 = min(tid * chunk, T), t1 = min(t0 + chunk, T);
-  // log2 classes of a heavy candidate (-1 otherwise) for the eight tiles
-  // from tb on, past t1 -2: their ranges are requested together (past the
-  // end a lane reads tile 0's and drops it) instead of one after another
-  constexpr uint32_t G = 8;
-  auto classes = [&](uint32_t tb, int (&c)[G]) {
-    uint2 r[G];
-#pragma unroll
-    for (uint32_t g = 0; g < G; ++g) r[g] = ranges[tb + g < t1 ? tb + g : 0u];
-#pragma unroll
-    for (uint32_t g = 0; g < G; ++g) {
-      const uint32_t len = r[g].y - r[g].x;
-      c[g] = tb + g >= t1 ? -2 : (len >= thr ? 31 - __clz(len) : -1);
-    }
-  };
-  for (uint32_t tb = t0; tb < t1; tb += G) {
-    int c[G];
-    classes(tb, c);
-#pragma unroll
-    for (uint32_t g = 0; g < G; ++g)
-      if (c[g] >= 0) atomicAdd(&s_cnt[c[g]], 1u);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    // whole classes, longest first, while they fit under the cap
-    uint32_t h = 0, cut = 32;
-    for (int c = 31; c >= 0; --c) {
-      if (h + s_cnt[c] > a.heavy_cap) break;
-      s_cur[c] = h;
-      h += s_cnt[c];
-      cut = (uint32_t)c;
-    }
-    s_cut = cut;
-    counters[kHeavyTiles] = h;
-    uint32_t split = 0;
-    if (a.split_mult) {
-      const uint32_t c_split = 31u - __clz(max(a.split_mult * mean, 2048u));
-      for (uint32_t c = max(c_split, cut); c < 32u; ++c) split += s_cnt[c];
-    }
-    counters[kSplitTiles] = split;
-  }
-  __syncthreads();
-  const uint32_t cut = s_cut;
-  uint32_t light = 0;
-  for (uint32_t tb = t0; tb < t1; tb += G) {
-    int c[G];
-    classes(tb, c);
-#pragma unroll
-    for (uint32_t g = 0; g < G; ++g) {
-      if (c[g] == -2) continue;
-      if (c[g] >= (int)cut) order[atomicAdd(&s_cur[c[g]], 1u)] = tb + g;
-      else ++light;
-    }
-  }
-  uint32_t total;
-  uint32_t pos = block_exclusive_scan<THREADS>(light, s_tmp, total);
-  const uint32_t heavy = T - total;
-  for (uint32_t tb = t0; tb < t1; tb += G) {
-    int c[G];
-    classes(tb, c);
-#pragma unroll
-    for (uint32_t g = 0; g < G; ++g)
-      if (c[g] != -2 && c[g] < (int)cut) order[heavy + pos++] = tb + g;
-  }
+  if (t >= T) return;
+  uint64_t pairs = 0;
+  for (int i = 0; i < a.views; ++i) pairs += min(a.counters[(size_t)i * kCounterWords + kPairs], a.pair_cap);
+  const uint32_t thr = max((uint32_t)min(pairs / kHeavyShare, (uint64_t)0x40000000u), kHeavyMin);
+  uint2* range = a.ranges + v * a.ranges_stride + t;
+  const uint2 r = *range;
+  const uint32_t len = r.y - r.x;
+  if (len < thr) return;
+  const uint32_t times = len / thr;
+  const uint32_t c = times >= 16u ? 3u : times >= 4u ? 2u : times >= 2u ? 1u : 0u;
+  uint32_t* const all = a.counters;  // one set of lists for all views, counted in view 0's block
+  if (atomicAdd(&all[kHeavyAll], 1u) >= a.heavy_cap) return;
+  const uint32_t at = atomicAdd(&all[kHeavyTiles + c], 1u);
+  a.list[c * kHeavyCap + at] = (v << 24) | t;
+  range->x = r.x | kHeavyFlag;
+  if (a.tile_work && v == 0) a.tile_work[t] = make_uint2(len, 0u);
 }
 
-void launch_tile_order(const OrderLaunch& a, hipStream_t s) {
-  hipLaunchKernelGGL(k_tile_order, dim3(1, a.views), dim3(1024), 0, s, a);
+void launch_heavy_tiles(const HeavyLaunch& a, hipStream_t s) {
+  hipLaunchKernelGGL(k_heavy_tiles, dim3((a.max_tiles + 255) / 256, a.views), dim3(256), 0, s, a);
 }
 
 // One 256-lane block per 16x16 tile; wave w owns the 8x8 quadrant
@@ -672,72 +439,50 @@ __global__ __launch_bounds__(256, MODE == 3 ? (B == 128 ? (F32 ? 6 : 7) : 5) : 1
   __shared__ __align__(16) uint32_t s_rows[LANES_ ? 4 : 1][LANES_ ? 64 : 4];
   __shared__ __align__(16) uint8_t s_sub[SUBS ? 4 : 1][SUBS ? 4 : 1][SUBS ? B : 4];  // mode 2: per 4x4 sub-block
 
-  // Block -> (view, tile).  First the heavy tiles of every view (their
-  // count rounded up to 8 blocks; with split_heavy, mode 3 only, four blocks
-  // per heavy tile, one per 8x8 quadrant, each wave two of its rows), then
-  // each view's other tiles in a slot range of slots_per_view blocks: blocks
-  // are dealt round-robin to the 8 XCDs, and the XCDs take runs of kXcdRun
-  // neighbouring tiles in turn (kXcdRun has why).  A heavy tile's pixels wait on their own long chains of
-  // blends; with one view on the device the other blocks are soon done, and
-  // sixteen waves on a tile instead of four shorten its chains' wave-wide
-  // steps (each step waits for the busiest of 16 pixels, not 64).
-  const uint32_t nv = (uint32_t)a.views;
-  uint32_t v = 0, pos = 0, quad = 4;  // quad < 4: the quadrant of a split heavy tile
-  {
-    uint32_t heavy_total = 0, split_total = 0;
-    if (a.longest_first)
-      for (uint32_t i = 0; i < nv; ++i) heavy_total += a.counters[(size_t)i * kCounterWords + kHeavyTiles];
-    // split tiles: the first of view 0's heavy tiles (splitting is for one view)
-    if (LANES && a.split_heavy && a.longest_first) split_total = a.counters[kSplitTiles];
-    const uint32_t split_blocks = ((split_total + 7u) & ~7u) * 4u;
-    const uint32_t heavy_blocks = split_blocks + ((heavy_total - split_total + 7u) & ~7u);
-    uint32_t b = blockIdx.x;
-    if (b < heavy_blocks) {
-      if (b < split_blocks) {
-        quad = b & 3u;
-        b >>= 2;
-        if (b >= split_total) return;
-      } else {
-        b = split_total + (b - split_blocks);
-        if (b >= heavy_total) return;
-      }
-      for (;; ++v) {
-        const uint32_t h = a.counters[(size_t)v * kCounterWords + kHeavyTiles];
-        if (b < h) break;
-        b -= h;
-      }
-      pos = b;
-    } else {
-      b -= heavy_blocks;
-      v = b / a.slots_per_view;
-      if (v >= nv) return;
-      const uint32_t k = b % a.slots_per_view;
-      const uint32_t p = ((k >> 3) / kXcdRun * 8u + (k & 7u)) * kXcdRun + (k >> 3) % kXcdRun;
-      const uint32_t h = a.longest_first ? a.counters[(size_t)v * kCounterWords + kHeavyTiles] : 0u;
-      const uint32_t tv = a.uniforms[v].tiles_x * a.uniforms[v].tiles_y;
-      if (p >= tv - h) return;
-      pos = h + p;
+  // Block -> (view, tile).  First eight blocks for each heavy tile, longest
+  // class first, then each view's tiles in a slot range of slots_per_view
+  // blocks.  Blocks are dealt round-robin to the 8 XCDs, and the XCDs take
+  // runs of kXcdRun neighbouring tiles in turn (kXcdRun has why).
+  uint32_t b = blockIdx.x;
+  const uint32_t heavy = min(a.counters[kHeavyAll], a.heavy_cap), heavy_blocks = 8u * ((heavy + 7u) & ~7u);
+  if (b < heavy_blocks) {
+    __shared__ __align__(16) uint32_t s_words[8];
+    // a tile's blocks on one XCD: they read the same records
+    uint32_t at = b / 64u * 8u + (b & 7u);
+    if (at >= heavy) return;
+    int c = kHeavyClasses - 1;
+    for (; c > 0; --c) {
+      const uint32_t h = a.counters[kHeavyTiles + c];
+      if (at < h) break;
+      at -= h;
     }
+    const uint32_t vt = a.heavy[c * kHeavyCap + at];
+    raster_heavy<UNALIGNED, F32>(a, vt >> 24, vt & 0xFFFFFFu, (b >> 3) & 7u, &s_ent[0][0][0], s_words);
+    return;
   }
+  b -= heavy_blocks;
+  const uint32_t v = b / a.slots_per_view;
+  if (v >= (uint32_t)a.views) return;
+  const uint32_t slot = b % a.slots_per_view;
+  const uint32_t tile = ((slot >> 3) / kXcdRun * 8u + (slot & 7u)) * kXcdRun + (slot >> 3) % kXcdRun;
+  if (tile >= a.uniforms[v].tiles_x * a.uniforms[v].tiles_y) return;
   const Uniforms& u = a.uniforms[v];
   const uint2* ranges = a.ranges + v * a.ranges_stride;
   const uint32_t* pair_vals = a.pair_vals + v * a.pair_stride;
   const float4* records = a.records + v * a.rec_stride;
-  const uint32_t tile = a.longest_first ? a.order[v * a.order_stride + pos] : pos;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-  // this wave's 8x8 region: quadrant w, or for a split tile rows 2w and
-  // 2w + 1 of quadrant quad (lanes 0-15; the others hold no pixel)
-  const uint32_t qd = quad < 4u ? quad : w;
-  const uint32_t qx0 = (tile % u.tiles_x) * kTileSize + (qd & 1u) * 8u;
-  const uint32_t qy0 = (tile / u.tiles_x) * kTileSize + (qd >> 1) * 8u + (quad < 4u ? 2u * w : 0u);
+  // this wave's 8x8 region: quadrant w
+  const uint32_t qx0 = (tile % u.tiles_x) * kTileSize + (w & 1u) * 8u;
+  const uint32_t qy0 = (tile / u.tiles_x) * kTileSize + (w >> 1) * 8u;
   // mode 2: lane group g = lane / 16 owns the 4x4 sub-block (g & 1, g >> 1)
   const uint32_t g = lane >> 4;
   const uint32_t px = SUBS ? qx0 + (g & 1u) * 4u + (lane & 3u) : qx0 + (lane & 7u);
   const uint32_t py = SUBS ? qy0 + (g >> 1) * 4u + ((lane >> 2) & 3u) : qy0 + (lane >> 3);
   const uint32_t W = u.image_size[0], H = u.image_size[1];
-  const bool inside = px < W && py < H && (quad == 4u || lane < 16u);
+  const bool inside = px < W && py < H;
   // (the ranges are cleared for the next frame by its pair sort)
   const uint2 range = ranges[tile];
+  if (range.x & kHeavyFlag) return;  // has blocks of its own
 
   const PixelMap pm = pixel_map(u);
   const float pxf = (float)px, pyf = (float)py;

@@ -23,7 +23,6 @@ using namespace spl;
 namespace {
 
 constexpr int kStageSlots = 4;  // pinned uniform uploads in flight
-constexpr uint32_t kSingleHeavyMult = 2;
 constexpr int kStageCount = 8;  // cull, histograms, sort, project, bin, pair sort, ranges, raster
 
 struct UploadSlot {
@@ -91,7 +90,7 @@ struct spl_renderer {
   uint32_t* depth_hist = nullptr;
   uint32_t* pair_hist = nullptr;
   uint2* ranges = nullptr;
-  uint32_t* tile_order = nullptr;  // per view, ranges_cap tiles
+  uint32_t* heavy = nullptr;  // k_heavy_tiles' lists
   uint32_t ranges_cap = 0;
   // shared
   uint32_t* vis = nullptr;
@@ -164,7 +163,7 @@ void renderer_free(spl_renderer* r) {
   dev_free(r->depth_hist);
   dev_free(r->pair_hist);
   dev_free(r->ranges);
-  dev_free(r->tile_order);
+  dev_free(r->heavy);
   dev_free(r->vis);
   dev_free(r->d_uniforms);
   dev_free(r->d_pixels);
@@ -243,16 +242,14 @@ int ensure_ranges(spl_renderer* r, uint32_t tiles) {
   HIP_TRY(hipStreamSynchronize(r->stream));
   drop_graph(r);
   dev_free(r->ranges);
-  dev_free(r->tile_order);
-  r->bytes -= (uint64_t)r->ranges_cap * r->max_views * (sizeof(uint2) + sizeof(uint32_t));
+  r->bytes -= (uint64_t)r->ranges_cap * r->max_views * sizeof(uint2);
   r->ranges_cap = 0;
   const size_t words = (size_t)tiles * r->max_views;
   HIP_TRY(dev_alloc(&r->ranges, words));
-  HIP_TRY(dev_alloc(&r->tile_order, words));
   HIP_TRY(hipMemsetAsync(r->ranges, 0, words * sizeof(uint2), r->stream));
   HIP_TRY(hipStreamSynchronize(r->stream));
   r->ranges_cap = tiles;
-  r->bytes += (uint64_t)words * (sizeof(uint2) + sizeof(uint32_t));
+  r->bytes += (uint64_t)words * sizeof(uint2);
   return SPL_OK;
 }
 
@@ -494,30 +491,23 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     launch_ranges(a, q);
   }
   const uint32_t slots = div_up(b.max_tiles, 8 * kXcdRun) * 8 * kXcdRun;
-  const uint32_t heavy_cap = std::max<uint32_t>(8, slots / 8);
-  // A single view rasters in 256-entry batches, its longest tiles first:
-  // with only one view's tiles on the device the longest ones set the
-  // frame's time (660.6 against 614.8 plain frames/s, 6M splats at 1080p on
-  // MI355X).  Batches of views keep the configured form, which suits
-  // throughput (the autotuner picks it).  Every form gives the same image.
-  const bool single = nv == 1;
-  const uint32_t raster_batch = single ? 256u : cfg.raster_batch;
-  const bool longest_first = single || cfg.raster_longest_first != 0;
-  if (longest_first) {
-    OrderLaunch a{};
+  // One view rasters in 128-entry batches: with its longest tiles on blocks of
+  // their own, seven blocks per CU beat the longer batches (6M splats at 1080p
+  // 1210 against 1277 us a frame, 1M 561 against 584).
+  const uint32_t raster_batch = nv == 1 ? 128u : cfg.raster_batch;
+  const uint32_t heavy_cap = std::min<uint32_t>(kHeavyCap, nv * b.max_tiles);
+  {
+    HeavyLaunch a{};
     a.ranges = r->ranges; a.ranges_stride = r->ranges_cap;
     a.uniforms = r->d_uniforms;
     a.counters = r->counters;
     a.pair_cap = (uint32_t)r->pair_cap;
-    a.order = r->tile_order; a.order_stride = r->ranges_cap;
+    a.list = r->heavy;
     a.heavy_cap = heavy_cap;
-    // one view: tiles from twice the mean list go first (its time is set by
-    // its longest tiles), those from 8x the mean on four blocks each
-    a.heavy_mult = single ? kSingleHeavyMult : 8u;
-    a.heavy_min = single ? 512u : 2048u;
-    a.split_mult = single && cfg.raster_mode == 3 ? 8u : 0u;
+    a.tile_work = b.tile_stats ? r->tile_work : nullptr;
+    a.max_tiles = b.max_tiles;
     a.views = (int)nv;
-    launch_tile_order(a, q);
+    launch_heavy_tiles(a, q);
   }
   mark(7);
   {
@@ -532,15 +522,12 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.blend_f32 = cfg.blend_mode == SPL_BLEND_F32 ? 1 : 0;
     a.walk = (int)cfg.raster_mode;
     a.batch_entries = (int)raster_batch;
-    a.longest_first = longest_first ? 1 : 0;
     a.bgra = cfg.frame_format == SPL_FRAME_FORMAT_BGRA8_UNORM ? 1 : 0;
     a.tile_work = b.tile_stats ? r->tile_work : nullptr;
-    a.order = r->tile_order; a.order_stride = r->ranges_cap;
+    a.heavy = r->heavy;
     a.slots_per_view = slots;
     a.heavy_cap = heavy_cap;
-    // one view in mode 3: each heavy tile's four quadrants go to four blocks
-    a.split_heavy = single && cfg.raster_mode == 3 ? 1 : 0;
-    a.grid_x = (int)(nv * slots + (longest_first ? ((nv * heavy_cap + 7) / 8) * 8 * (a.split_heavy ? 5 : 1) : 0));
+    a.grid_x = (int)(8 * div_up(heavy_cap, 8) * 8 + nv * slots);
     a.views = (int)nv;
     launch_raster(a, q);
   }
@@ -757,11 +744,12 @@ int renderer_create(spl_device* dev, const spl_configuration* cfg, bool own_stre
   chk(alloc(&r->counters, V * kCounterWords));
   chk(alloc(&r->depth_hist, V * kMaxDepthPasses * 1024));
   chk(alloc(&r->pair_hist, V * kMaxPairPasses * 256));
+  chk(alloc(&r->heavy, (size_t)kHeavyClasses * kHeavyCap));
   chk(alloc(&r->vis, r->cap));
   chk(alloc(&r->d_uniforms, V));
   chk(alloc(&r->d_pixels, V));
   if (dry) {
-    *dry_bytes = r->bytes + (uint64_t)presize_tiles * V * (sizeof(uint2) + sizeof(uint32_t));
+    *dry_bytes = r->bytes + (uint64_t)presize_tiles * V * sizeof(uint2);
     delete r;
     return SPL_OK;
   }
@@ -846,7 +834,7 @@ int render_frame_scratch(spl_device* dev, const spl_configuration* cfg, spl_scen
     take(&r.compact_idx, r.cap);
     take(&r.records, r.cap * kRecordFloat4);
     take(&r.boxes, r.cap);
-    take(&r.tile_order, tiles);
+    take(&r.heavy, (uint64_t)kHeavyClasses * kHeavyCap);
     for (int i = 0; i < 2; ++i) {
       take(&r.pair_keys[i], r.pair_cap);
       take(&r.pair_vals[i], r.pair_cap);

@@ -50,10 +50,23 @@ enum CounterSlot : int {
   kPairs = 33,
   kPairOverflow = 34,
   kScatterError = 35,
-  kHeavyTiles = 36, // tiles the raster takes first (longest lists)
-  kSplitTiles = 37, // the first of those, that the raster splits over four blocks
+  kHeavyAll = 36,   // view 0's block: tiles that k_heavy_tiles found heavy
+  kHeavyTiles = 37, // .. + kHeavyClasses - 1: tiles in each of its lists
   kCounterWords = 64
 };
+
+// Heavy tiles: lists of at least kHeavyMin pairs and 1 / kHeavyShare of the
+// batch's pairs (so never more than kHeavyCap of them).  An ordinary block
+// takes about 11 ns for each entry of its list, the device about 25 entries a
+// ns over all tiles: a list of 1/275 of the pairs lasts as long as the whole
+// raster.  The share is some four times that, because a frame saturates most
+// tiles early and the long lists cluster on screen; us a pass at 1/400, 1/900,
+// 1/1400 and 1/2500: 6M splats at 1080p 1180, 1127, 1090, 1549; 1M 540, 530,
+// 525, 598; 1.5M at VGA 462, 455, 467, 465; five views of 300k 575, 535, 537,
+// 665 (at 1/2500 they are too many for the eightfold reading to pay).
+constexpr uint32_t kHeavyShare = 1000, kHeavyMin = 512, kHeavyCap = 1000;
+constexpr int kHeavyClasses = 4;
+constexpr uint32_t kHeavyFlag = 0x80000000u;  // in a tile range's start (starts are below 2^30)
 
 // Scene data in HBM, one stream per attribute (structure of arrays).
 struct SceneView {
@@ -171,22 +184,22 @@ struct RangesLaunch {
   int grid_x, views;
 };
 
-struct OrderLaunch {
-  const uint2* ranges; size_t ranges_stride;
+struct HeavyLaunch {
+  uint2* ranges; size_t ranges_stride;
   const Uniforms* uniforms;
   uint32_t* counters;
   uint32_t pair_cap;
-  uint32_t* order; size_t order_stride;      // per view: heavy tiles, longest first, then the rest in order
-  uint32_t heavy_cap;                        // at most this many heavy tiles per view
-  uint32_t heavy_mult, heavy_min;            // heavy: at least heavy_mult x the mean and heavy_min pairs
-  uint32_t split_mult;                       // split: at least split_mult x the mean and 2048 pairs (0: none)
+  uint32_t* list;                            // kHeavyClasses lists of kHeavyCap: view << 24 | tile
+  uint32_t heavy_cap;                        // most tiles listed: kHeavyCap, or all tiles
+  uint2* tile_work;                          // optional, view 0, as in RasterLaunch
+  uint32_t max_tiles;
   int views;
 };
 
 struct RasterLaunch {
-  const uint32_t* order; size_t order_stride;
-  uint32_t slots_per_view;   // multiple of 8 * kXcdRun, >= the largest view's tile count
+  const uint32_t* heavy;     // k_heavy_tiles' lists
   uint32_t heavy_cap;
+  uint32_t slots_per_view;   // multiple of 8 * kXcdRun, >= the largest view's tile count
   const uint32_t* pair_vals; size_t pair_stride;
   const float4* records; size_t rec_stride;
   uint2* ranges; size_t ranges_stride;
@@ -198,8 +211,6 @@ struct RasterLaunch {
   int walk;                  // raster mode: 0 entry-major per quadrant, 1 per-pixel walk, 2 per 4x4 sub-block,
                              // 3 per-lane walk over coverage masks
   int batch_entries;         // entries staged in LDS per batch: 128 or 256
-  int longest_first;         // take the tiles in the order k_tile_order wrote
-  int split_heavy;           // mode 3, longest first: a heavy tile's quadrants on four blocks, two rows a wave
   int bgra;
   uint2* tile_work;          // optional, view 0: per tile (list length, entries consumed)
   int grid_x, views;
@@ -211,7 +222,7 @@ void launch_sort_pass(int bits, const SortPassLaunch& a, hipStream_t s);
 void launch_project(const ProjectLaunch& a, hipStream_t s);
 void launch_bin(const BinLaunch& a, hipStream_t s);
 void launch_ranges(const RangesLaunch& a, hipStream_t s);
-void launch_tile_order(const OrderLaunch& a, hipStream_t s);
+void launch_heavy_tiles(const HeavyLaunch& a, hipStream_t s);
 void launch_raster(const RasterLaunch& a, hipStream_t s);
 
 // spl_render_frame_static: the scratch array's size and the largest scene and

@@ -88,3 +88,39 @@ def test_sort_tile_of_one_view(count, bits):
     batch = frames[0].read()
     r.render_frame(frames[0], cam, view, scene)
     assert np.array_equal(frames[0].read(), batch)
+
+
+# A list of 512 pairs and 1/1000 of the frame's makes a tile heavy.  Lists from
+# one below that to a few batches of 128 and chunks of 64 entries more, in
+# whole and cut sub-blocks, that stay transparent or turn opaque on the way.
+@pytest.mark.parametrize("count,logit", [(511, -4.0), (512, -4.0), (513, -4.0), (640, -4.0), (641, -6.0), (1000, -4.0),
+                                         (5000, -6.0), (5000, 0.0), (5000, 6.0)])
+@pytest.mark.parametrize("width,height", [(16, 16), (13, 5), (21, 18)])
+@pytest.mark.parametrize("unaligned,blend", [(True, sa.BlendMode.UNORM8), (False, sa.BlendMode.F32),
+                                             (True, sa.BlendMode.F32), (False, sa.BlendMode.UNORM8)])
+def test_heavy_tiles(count, logit, width, height, unaligned, blend):
+    say(f"{count} splats, opacity logit {logit}, {width}x{height}, unaligned {unaligned}, blend {blend}")
+    case = Case(Workload("gaussian", 0, seed=0),
+                config(max_splat_count=count, max_views=2, use_unaligned_rectangles=unaligned, blend_mode=blend,
+                       tile_pairs_per_splat=8), width, height, sphere_pose(51, radius=5))
+    rec = Workload("gaussian", count, seed=51).all()
+    rec["center"] *= 0.1  # in front of the camera, all in the first tile of a 16x16 frame
+    rec["scale"] += 2.0   # a few pixels each
+    rec["alpha"] = logit
+    case.records, case.splats = rec, ob.decode(rec)
+    case.scene = sa.Scene(case.renderer, count)
+    case.scene.load_records(0, rec)
+    case.renderer.enable_tile_stats(True)
+    img = case.render()
+    lens = case.renderer.tile_stats()
+    say(f"  lists {lens[:, 0].tolist()}, consumed {lens[:, 1].tolist()}")
+    if (width, height) == (16, 16):
+        assert lens[0, 0] == count  # the list the case is about
+    assert (lens[:, 1] <= lens[:, 0] + 127).all()
+    _, _, _, oimg = case.oracle()
+    assert image_diff(img, oimg) <= IMAGE_TOL
+    # the same view in a batch, whose other view has lists of its own
+    other = sa.Frame(device(), 40, 24)
+    case.renderer.render_views([case.frame, other], [case.cam] * 2, [case.view] * 2, case.scene)
+    got = case.frame.read()
+    assert np.array_equal(got[..., [2, 1, 0, 3]] if case.cfg.frame_format == sa.FrameFormat.BGRA8_UNORM else got, img)
