@@ -150,6 +150,7 @@ __global__ __launch_bounds__(THREADS) void k_cull_views(CullLaunch a) {
         }
       }
     }
+    if (one_tile_each(num_tiles)) break;
     __syncthreads();
   }
 }

@@ -336,6 +336,7 @@ __global__ __launch_bounds__(THREADS) void k_bin(BinLaunch a) {
       }
     }
     __syncthreads();
+    if (one_tile_each(num_tiles)) break;
   }
   for (int i = tid; i < a.pair_passes * 256; i += THREADS)
     if (s_hist[i]) atomicAdd(&a.hist[v * a.hist_stride + i], s_hist[i]);

@@ -258,6 +258,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     const uint32_t left = n - t * TILE;
     if (left >= (uint32_t)TILE) tile_pass(Flag<true>{}, t, (uint32_t)TILE);
     else tile_pass(Flag<false>{}, t, left);
+    if (one_tile_each(num_tiles)) break;
   }
 }
 

@@ -172,19 +172,22 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
 // Tickets of a persistent grid.  Blocks take tiles in order from a counter:
 // an atomic on one address costs about 11.5 ns however many blocks issue it
 // (1024 tickets 11.8 us, measured), so a launch spends as few as it can.
-// Blocks past the number of tiles leave without a ticket, and every other
-// block's last ticket is past the tiles, which makes num_tiles + active
-// tickets in all: whoever draws the last one resets the counter for the next
-// launch.  No second counter and no fence: the tickets before the last have
-// been drawn, and the launch's end publishes the reset.  (A counter of
+// Blocks past the number of tiles leave without a ticket.  Where every tile
+// has a block, each of those draws one and is done (a second ticket would cost
+// a block another microsecond to learn that there are no more); otherwise
+// every block's last ticket is past the tiles.  Either way the number of
+// tickets is known, and whoever draws the last one resets the counter for the
+// next launch.  No second counter and no fence: the tickets before the last
+// have been drawn, and the launch's end publishes the reset.  (A counter of
 // leaving blocks behind a __threadfence, which writes an XCD's L2 back, cost
 // 1024 blocks 20 to 40 us.)
 __device__ __forceinline__ bool persistent_idle(uint32_t num_tiles) { return blockIdx.x >= num_tiles; }
+__device__ __forceinline__ bool one_tile_each(uint32_t num_tiles) { return gridDim.x >= num_tiles; }
 
 __device__ __forceinline__ uint32_t take_ticket(uint32_t* counter, uint32_t num_tiles) {
   const uint32_t t = atomicAdd(counter, 1u);
-  const uint32_t active = gridDim.x < num_tiles ? gridDim.x : num_tiles;
-  if (t == num_tiles + active - 1u) atomicExch(counter, 0u);
+  const uint32_t tickets = one_tile_each(num_tiles) ? num_tiles : num_tiles + gridDim.x;
+  if (t == tickets - 1u) atomicExch(counter, 0u);
   return t;
 }
 
