@@ -315,6 +315,8 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   const bool fork = sorted && !ev && r->side != nullptr;
   auto clampg = [](uint64_t want, uint32_t hi) { return (int)std::max<uint64_t>(1, std::min<uint64_t>(want, hi)); };
 
+  const bool cull_hist = sorted && nv == 1;  // the cull counts one view's digits itself
+
   mark(0);
   {
     CullLaunch a{};
@@ -330,7 +332,9 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.tile_prefix = r->tile_prefix; a.tp_stride = r->cull_tiles;
     a.status = r->cull_status; a.status_stride = r->cull_tiles;
     a.counters = r->counters;
-    a.grid = clampg(div_up(n, kCullTile), cus * 4);
+    a.hist = cull_hist ? r->depth_hist : nullptr;
+    a.bits = bits;
+    a.grid = clampg(div_up(n, kCullTile), cus * 2);  // two resident 1024-lane blocks per CU
     launch_cull(a, q);
   }
   auto launch_proj = [&](hipStream_t qq) {
@@ -346,7 +350,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.records = r->records; a.rec_stride = cap * kRecordFloat4;
     a.boxes = r->boxes; a.box_stride = cap;
     a.conics = b.conics ? r->conics : nullptr;
-    if (P == 0) {  // (sorted, the histograms clear the cull's words and the binning the sort's)
+    if (P == 0) {  // (sorted, the histograms or the first pass clear the cull's words and the binning the sort's)
       a.clear_a = r->cull_status;
       a.clear_a_words = cull_used;
       a.clear_a_stride = r->cull_tiles;
@@ -369,7 +373,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     launch_proj(r->side);
     (void)hipEventRecord(r->join, r->side);
   }
-  if (sorted) {
+  if (sorted && !cull_hist) {
     HistLaunch a{};
     a.keys = r->keys[0]; a.keys_stride = cap;
     a.hist = r->depth_hist; a.hist_stride = (size_t)kMaxDepthPasses * 1024;
@@ -400,6 +404,10 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a = r->sort_status + (size_t)(p - 1) * r->sort_words;
       a.clear_a_words = sort_used;
       a.clear_a_stride = sort_stride;
+    } else if (cull_hist) {
+      a.clear_a = r->cull_status;
+      a.clear_a_words = cull_used;
+      a.clear_a_stride = r->cull_tiles;
     }
     a.threads = depth_threads;
     a.grid_x = sort_grid(n, depth_threads);

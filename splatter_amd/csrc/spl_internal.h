@@ -107,6 +107,8 @@ struct CullLaunch {
   uint32_t* tile_prefix; size_t tp_stride;   // [views][cull tiles] exclusive prefix
   uint32_t* status; size_t status_stride;    // [views][cull tiles]
   uint32_t* counters;                        // [views][kCounterWords]
+  uint32_t* hist;                            // one view: [passes << bits] digit histograms; null: not here
+  int bits;
   int grid;
 };
 
