@@ -168,12 +168,9 @@ __global__ __launch_bounds__(THREADS) void k_cull_views(CullLaunch a) {
       }
     }
     if (one_tile_each(num_tiles)) break;
-<<<<<<< Updated upstream
-=======
     __syncthreads();
   }
   if constexpr (BITS > 0) {
->>>>>>> Stashed changes
     __syncthreads();
     for (int i = tid; i < PASSES * RADIX; i += THREADS) {
       uint32_t sum = 0;
