@@ -176,7 +176,7 @@ __global__ __launch_bounds__(THREADS) void k_cull_views(CullLaunch a) {
       uint32_t sum = 0;
 #pragma unroll
       for (int r = 0; r < REP; ++r) sum += s_hist[i * REP + r];
-      if (sum) atomicAdd(&a.hist[i], sum);
+      if (sum) atomicAdd(&a.hist[(blockIdx.x % kHistCopies) * a.hist_copy + i], sum);
     }
   }
 }

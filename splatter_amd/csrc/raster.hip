@@ -161,24 +161,26 @@ __device__ __forceinline__ void walk_run(const float4* cm, const float4* ct, con
 
 }  // namespace
 
+// Bound by the latency of a tile's chain (ticket, box gather, look-back) in
+// small frames and by the expansion's LDS reads and VALU in large ones.  Each
+// entry of the tile is one 16-byte LDS row (first output slot, first screen
+// tile and width packed, record), stored item-major so that a wave writes
+// consecutive rows; logical entry i = 4 tid + k (ITEMS = 4) is row
+// k * THREADS + tid.  Tiles of more than 4096 pairs expand through the owner
+// table 4096 slots at a time (a binary search over the offsets, ten dependent
+// LDS reads a pair, took 61 us on 100k splats at 720p, which take 16 now; 8
+// views of 32M at 4K render in 65.7 ms instead of 70.5).
 template <int THREADS, int ITEMS>
 __global__ __launch_bounds__(THREADS) void k_bin(BinLaunch a) {
   constexpr int TILE = THREADS * ITEMS;
   constexpr int WAVES = THREADS / kWave;
-  static_assert(ITEMS == 4, "a thread's items are one 16-byte LDS row");
-  // Per entry of the tile: first output slot, first tile (x | y << 16),
-  // width in tiles, record.  Thread t's four entries are one 16-byte row of
-  // each array, written with one store (consecutive threads, consecutive
-  // banks; four separate words a thread would put 8 lanes on each bank).
-  __shared__ __align__(16) uint32_t s_off[TILE + 4];
-  __shared__ __align__(16) uint32_t s_org[TILE];
-  __shared__ __align__(16) uint32_t s_w[TILE];
-  __shared__ __align__(16) uint32_t s_rec[TILE];
-  // the entry that owns each output slot of a tile with at most OWN pairs
+  constexpr int REP = 2;  // histogram copies across lanes: neighbouring pairs share their high digit
+  __shared__ uint4 s_ent[TILE];
+  // the entry that owns each of OWN output slots
   constexpr uint32_t OWN = 4096, PER = OWN / THREADS;
   static_assert(PER == 16, "a thread's owner slots are two 16-byte LDS rows");
   __shared__ __align__(16) uint16_t s_own[OWN];
-  __shared__ uint32_t s_hist[kMaxPairPasses * 256];
+  __shared__ uint32_t s_hist[kMaxPairPasses * 256 * REP];
   __shared__ uint32_t s_tmp[WAVES];
   __shared__ uint32_t s_tile;
   __shared__ uint64_t s_prefix;
@@ -193,7 +195,7 @@ __global__ __launch_bounds__(THREADS) void k_bin(BinLaunch a) {
   uint64_t* status = a.status + v * a.status_stride;
   if (a.clear_a) clear_words(a.clear_a + v * a.clear_a_stride, a.clear_a_words);
   if (a.clear_b) clear_words(a.clear_b + v * a.clear_b_stride, a.clear_b_words);
-  for (int i = tid; i < a.pair_passes * 256; i += THREADS) s_hist[i] = 0u;
+  for (int i = tid; i < a.pair_passes * 256 * REP; i += THREADS) s_hist[i] = 0u;
   const uint32_t n = counters[kVisible];
   const uint32_t num_tiles = (n + TILE - 1) / TILE;
   if (num_tiles == 0 && blockIdx.x == 0 && tid == 0) {
@@ -225,13 +227,15 @@ __global__ __launch_bounds__(THREADS) void k_bin(BinLaunch a) {
       if (r >= n || rec[k] >= n) rec[k] = 0u;  // never read past the boxes
       box[k] = boxes[rec[k]];
     }
-    uint32_t org[ITEMS], wid[ITEMS], off[ITEMS];
+    // screen tiles up to 1024 across and down (frames up to 16384 pixels):
+    // x, y and the width of at most 1024 pack into 31 bits
+    static_assert(kTileSize == 16, "tile coordinates in 10 bits");
+    uint32_t geom[ITEMS], off[ITEMS];
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const uint32_t r = t * TILE + tid * ITEMS + k;
       cnt[k] = 0;
-      org[k] = 0;
-      wid[k] = 0;
+      geom[k] = 1u << 20;
       if (r < n) {
         const uint2 q = box[k];
         const uint32_t lo = q.x, hi = q.y;
@@ -239,54 +243,42 @@ __global__ __launch_bounds__(THREADS) void k_bin(BinLaunch a) {
         const uint32_t x1 = (hi & 0xFFFFu) / kTileSize, y1 = (hi >> 16) / kTileSize;
         if (lo != 0xFFFFFFFFu && x1 >= x0 && y1 >= y0) {
           cnt[k] = (x1 - x0 + 1) * (y1 - y0 + 1);
-          org[k] = x0 | (y0 << 16);
-          wid[k] = x1 - x0 + 1;
+          geom[k] = x0 | (y0 << 10) | ((x1 - x0 + 1) << 20);
         }
       }
       sum += cnt[k];
     }
-    // (an entry without pairs owns no slot, so its row is never read)
-    reinterpret_cast<uint4*>(s_org)[tid] = make_uint4(org[0], org[1], org[2], org[3]);
-    reinterpret_cast<uint4*>(s_w)[tid] = make_uint4(wid[0], wid[1], wid[2], wid[3]);
-    reinterpret_cast<uint4*>(s_rec)[tid] = make_uint4(rec[0], rec[1], rec[2], rec[3]);
     uint32_t total;
     uint32_t excl = block_exclusive_scan<THREADS>(sum, s_tmp, total);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       off[k] = excl;
+      s_ent[k * THREADS + tid] = make_uint4(excl, geom[k], rec[k], 0u);
       excl += cnt[k];
     }
-    reinterpret_cast<uint4*>(s_off)[tid] = make_uint4(off[0], off[1], off[2], off[3]);
     if (tid < kWave) {
       const uint64_t prefix = wave_lookback64(status, t, (uint64_t)total);
-      if (tid == 0) {
-        s_off[TILE] = total;
-        s_prefix = prefix;
-      }
+      if (tid == 0) s_prefix = prefix;
       if (tid == 0 && t == num_tiles - 1) {
         const uint64_t k_all = prefix + total;
         counters[kPairs] = (uint32_t)(k_all < a.pair_cap ? k_all : a.pair_cap);
         counters[kPairOverflow] = k_all > a.pair_cap ? 1u : 0u;
       }
     }
-    __syncthreads();
-    const uint64_t prefix = s_prefix;
-    // Owner of each output slot: every entry with pairs writes its index at
-    // its first slot, then an inclusive max-scan over the slots carries it
-    // forward, so the expansion reads a slot's owner instead of
-    // binary-searching the offsets (ten dependent LDS reads).  A tile with
-    // more than OWN pairs searches.
-    // (Slots past the total hold stale owners: the scan carries them only
-    // forward, into slots that no pair reads.)
-    const bool table = total <= OWN;
-    if (table) {
-      const uint32_t lane = tid & (kWave - 1), wv = tid / kWave;
-      uint4* const own4 = reinterpret_cast<uint4*>(s_own);  // eight slots a row
-      for (uint32_t q = tid; q < (total + 7u) / 8u; q += THREADS) own4[q] = make_uint4(0u, 0u, 0u, 0u);
+    // Output slots, OWN at a time.  Owner of each: every entry with pairs in
+    // them writes its index at its first, then an inclusive max-scan carries
+    // the indices forward.  (Slots past the last hold stale owners: the scan
+    // carries them only forward, into slots that no pair reads.)
+    const uint32_t lane = tid & (kWave - 1), wv = tid / kWave;
+    uint4* const own4 = reinterpret_cast<uint4*>(s_own);  // eight slots a row
+    for (uint32_t s0 = 0; s0 < total; s0 += OWN) {
+      const uint32_t m = min(total - s0, OWN);
+      for (uint32_t q = tid; q < (m + 7u) / 8u; q += THREADS) own4[q] = make_uint4(0u, 0u, 0u, 0u);
       __syncthreads();
 #pragma unroll
       for (int k = 0; k < ITEMS; ++k)
-        if (cnt[k] > 0u) s_own[off[k]] = (uint16_t)(tid * ITEMS + k);
+        if (cnt[k] > 0u && off[k] + cnt[k] > s0 && off[k] < s0 + OWN)
+          s_own[max(off[k], s0) - s0] = (uint16_t)(tid * ITEMS + k);
       __syncthreads();
       // this thread's sixteen slots, two rows; slot 2i + h is half h of word i
       const uint4 ra = own4[2 * tid], rb = own4[2 * tid + 1];
@@ -314,32 +306,39 @@ __global__ __launch_bounds__(THREADS) void k_bin(BinLaunch a) {
       own4[2 * tid] = make_uint4(wd[0], wd[1], wd[2], wd[3]);
       own4[2 * tid + 1] = make_uint4(wd[4], wd[5], wd[6], wd[7]);
       __syncthreads();
-    }
-    for (uint32_t s = tid; s < total; s += THREADS) {
-      uint32_t lo = 0, hi = TILE - 1;
-      if (table) {
-        lo = s_own[s];
-      } else {
-        while (lo < hi) {
-          const uint32_t mid = (lo + hi + 1) >> 1;
-          if (s_off[mid] <= s) lo = mid; else hi = mid - 1;
+      const uint64_t prefix = s_prefix + s0;
+      for (uint32_t s = tid; s < m; s += THREADS) {
+        const uint32_t lo = s_own[s];
+        const uint4 e = s_ent[lo % ITEMS * THREADS + lo / ITEMS];
+        const uint64_t pos = prefix + s;
+        if (pos < a.pair_cap) {
+          // row and column of pair k in a box w tiles wide: (k + 1/2) / w is
+          // at least 1/2w from an integer, and the product's error is below
+          // (k + 1/2) / w * 2^-22, so its floor is k / w for k < 2^20
+          const uint32_t k = s0 + s - e.x, w = e.y >> 20;
+          const uint32_t row = (uint32_t)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)w));
+          const uint32_t tile = (((e.y >> 10) & 1023u) + row) * tiles_x + (e.y & 1023u) + (k - row * w);
+          pair_keys[pos] = tile;
+          pair_vals[pos] = e.z;
+          for (int q = 0; q < a.pair_passes; ++q)
+            atomicAdd(&s_hist[(q * 256 + ((tile >> (8 * q)) & 255u)) * REP + (tid & (REP - 1))], 1u);
         }
       }
-      const uint64_t pos = prefix + s;
-      if (pos < a.pair_cap) {
-        const uint32_t k = s - s_off[lo];
-        const uint32_t w = s_w[lo], org = s_org[lo];
-        const uint32_t tile = ((org >> 16) + k / w) * tiles_x + (org & 0xFFFFu) + k % w;
-        pair_keys[pos] = tile;
-        pair_vals[pos] = s_rec[lo];
-        for (int q = 0; q < a.pair_passes; ++q) atomicAdd(&s_hist[q * 256 + ((tile >> (8 * q)) & 255u)], 1u);
-      }
+      __syncthreads();
     }
-    __syncthreads();
     if (one_tile_each(num_tiles)) break;
+    __syncthreads();
   }
-  for (int i = tid; i < a.pair_passes * 256; i += THREADS)
-    if (s_hist[i]) atomicAdd(&a.hist[v * a.hist_stride + i], s_hist[i]);
+  __syncthreads();
+  // each XCD's blocks add to a copy of their own: an address that every block
+  // adds to takes 11.5 ns a block
+  uint32_t* hist = a.hist + v * a.hist_stride + (blockIdx.x % kHistCopies) * (kMaxPairPasses * 256);
+  for (int i = tid; i < a.pair_passes * 256; i += THREADS) {
+    uint32_t c = 0;
+#pragma unroll
+    for (int r = 0; r < REP; ++r) c += s_hist[i * REP + r];
+    if (c) atomicAdd(&hist[i], c);
+  }
 }
 
 // Run boundaries of the tile-sorted pair keys, four keys per thread.
@@ -719,7 +718,9 @@ __global__ __launch_bounds__(256, MODE == 3 ? (B == 128 ? (F32 ? 6 : 7) : 5) : 1
 }
 
 void launch_bin(const BinLaunch& a, hipStream_t s) {
-  hipLaunchKernelGGL((k_bin<kBinThreads, kBinItems>), dim3(a.grid_x, a.views), dim3(kBinThreads), 0, s, a);
+  const dim3 grid(a.grid_x, a.views), block(kBinThreads);
+  if (a.items == 1) hipLaunchKernelGGL((k_bin<kBinThreads, 1>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((k_bin<kBinThreads, kBinItems>), grid, block, 0, s, a);
 }
 
 void launch_ranges(const RangesLaunch& a, hipStream_t s) {

@@ -23,6 +23,7 @@ using namespace spl;
 namespace {
 
 constexpr int kStageSlots = 4;  // pinned uniform uploads in flight
+constexpr size_t kDepthHist = (size_t)kMaxDepthPasses * 1024, kPairHist = (size_t)kMaxPairPasses * 256;  // words a copy
 constexpr int kStageCount = 8;  // cull, histograms, sort, project, bin, pair sort, ranges, raster
 
 struct UploadSlot {
@@ -315,6 +316,11 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   const bool fork = sorted && !ev && r->side != nullptr;
   auto clampg = [](uint64_t want, uint32_t hi) { return (int)std::max<uint64_t>(1, std::min<uint64_t>(want, hi)); };
 
+  // Bin tiles of 256 entries where that puts more CUs at work, of 1024 where
+  // the tickets (11.5 ns each) and the look-back over many tiles cost more;
+  // us in tiles of 256 / 1024: 20k splats 10.6 / 12.7, 100k at 720p 16 / 27,
+  // 400k 22 / 14, 1M 46 / 25.
+  const int bin_items = (uint64_t)n * nv <= 1u << 17 ? 1 : kBinItems;
   const bool cull_hist = sorted && nv == 1;  // the cull counts one view's digits itself
 
   mark(0);
@@ -333,6 +339,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.status = r->cull_status; a.status_stride = r->cull_tiles;
     a.counters = r->counters;
     a.hist = cull_hist ? r->depth_hist : nullptr;
+    a.hist_copy = kDepthHist;
     a.bits = bits;
     a.grid = clampg(div_up(n, kCullTile), cus * 2);  // two resident 1024-lane blocks per CU
     launch_cull(a, q);
@@ -376,7 +383,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   if (sorted && !cull_hist) {
     HistLaunch a{};
     a.keys = r->keys[0]; a.keys_stride = cap;
-    a.hist = r->depth_hist; a.hist_stride = (size_t)kMaxDepthPasses * 1024;
+    a.hist = r->depth_hist; a.hist_stride = kHistCopies * kDepthHist;
     a.counters = r->counters;
     a.passes = P;
     a.bits = bits;
@@ -397,7 +404,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.count_slot = kVisible;
     a.count_cap = n;
     a.shift = p * bits;
-    a.hist = r->depth_hist + (size_t)p * radix; a.hist_stride = (size_t)kMaxDepthPasses * 1024;
+    a.hist = r->depth_hist + (size_t)p * radix; a.hist_stride = kHistCopies * kDepthHist; a.hist_copy = kDepthHist;
     a.status = r->sort_status + (size_t)p * r->sort_words; a.status_stride = sort_stride;
     a.tile_slot = kCtrSort0 + p;
     if (p > 0) {
@@ -427,8 +434,8 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_words = sort_used;
       a.clear_a_stride = sort_stride;
       a.clear_b = r->depth_hist;
-      a.clear_b_words = (size_t)kMaxDepthPasses * 1024;
-      a.clear_b_stride = (size_t)kMaxDepthPasses * 1024;
+      a.clear_b_words = kHistCopies * kDepthHist;
+      a.clear_b_stride = kHistCopies * kDepthHist;
     }
     a.order = sorted ? r->vals[fin] : nullptr; a.order_stride = cap;
     a.boxes = r->boxes; a.box_stride = cap;
@@ -436,11 +443,12 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.pair_keys = r->pair_keys[0];
     a.pair_vals = r->pair_vals[0]; a.pair_stride = r->pair_cap;
     a.pair_cap = (uint32_t)r->pair_cap;
-    a.hist = r->pair_hist; a.hist_stride = (size_t)kMaxPairPasses * 256;
+    a.hist = r->pair_hist; a.hist_stride = kHistCopies * kPairHist;
     a.pair_passes = Q;
     a.status = r->bin_status; a.status_stride = r->bin_words;
     a.counters = r->counters;
-    a.grid_x = clampg(div_up(n, kBinThreads * kBinItems), per_view);
+    a.items = bin_items;
+    a.grid_x = clampg(div_up(n, kBinThreads * bin_items), per_view);
     a.views = (int)nv;
     launch_bin(a, q);
   }
@@ -456,12 +464,12 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.count_slot = kPairs;
     a.count_cap = (uint32_t)r->pair_cap;
     a.shift = 8 * p;
-    a.hist = r->pair_hist + (size_t)p * 256; a.hist_stride = (size_t)kMaxPairPasses * 256;
+    a.hist = r->pair_hist + (size_t)p * 256; a.hist_stride = kHistCopies * kPairHist; a.hist_copy = kPairHist;
     a.status = r->pair_status + (size_t)p * r->pair_words; a.status_stride = pair_stride_status;
     a.tile_slot = kCtrPair0 + p;
     if (p == 0) {
       a.clear_a = reinterpret_cast<uint32_t*>(r->bin_status);
-      a.clear_a_words = (size_t)div_up(n, kBinThreads * kBinItems) * 2;
+      a.clear_a_words = (size_t)div_up(n, kBinThreads * bin_items) * 2;
       a.clear_a_stride = r->bin_words * 2;
       // the tile ranges the previous frame's raster read: tiles without
       // pairs in this frame must read as empty
@@ -492,8 +500,8 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.clear_a_words = r->pair_words;
     a.clear_a_stride = pair_stride_status;
     a.clear_b = r->pair_hist;
-    a.clear_b_words = (size_t)kMaxPairPasses * 256;
-    a.clear_b_stride = (size_t)kMaxPairPasses * 256;
+    a.clear_b_words = kHistCopies * kPairHist;
+    a.clear_b_stride = kHistCopies * kPairHist;
     a.grid_x = clampg(div_up(r->pair_cap, 1024), std::max<uint32_t>(1, cus * 32 / nv));
     a.views = (int)nv;
     launch_ranges(a, q);
@@ -703,7 +711,7 @@ void size_workspace(spl_renderer* r, const spl_configuration* cfg, uint64_t cap,
   if (r->pair_cap == 0) r->pair_cap = 4;
   r->cull_tiles = div_up(r->cap, kCullTile);
   r->sort_words = (size_t)div_up(r->cap, kSortThreads * kSortItems) * radix;
-  r->bin_words = div_up(r->cap, kBinThreads * kBinItems);
+  r->bin_words = div_up(r->cap, kBinThreads);
   r->pair_words = (size_t)div_up(r->pair_cap, kSortThreads * kSortItems) * 256;
 }
 
@@ -750,8 +758,8 @@ int renderer_create(spl_device* dev, const spl_configuration* cfg, bool own_stre
   chk(alloc(&r->bin_status, V * r->bin_words));
   chk(alloc(&r->pair_status, V * r->pair_words * kMaxPairPasses));
   chk(alloc(&r->counters, V * kCounterWords));
-  chk(alloc(&r->depth_hist, V * kMaxDepthPasses * 1024));
-  chk(alloc(&r->pair_hist, V * kMaxPairPasses * 256));
+  chk(alloc(&r->depth_hist, V * kHistCopies * kDepthHist));
+  chk(alloc(&r->pair_hist, V * kHistCopies * kPairHist));
   chk(alloc(&r->heavy, (size_t)kHeavyClasses * kHeavyCap));
   chk(alloc(&r->vis, r->cap));
   chk(alloc(&r->d_uniforms, V));
@@ -777,8 +785,8 @@ int renderer_create(spl_device* dev, const spl_configuration* cfg, bool own_stre
     chk(hipMemsetAsync(r->bin_status, 0, V * r->bin_words * 8, r->stream));
     chk(hipMemsetAsync(r->pair_status, 0, V * r->pair_words * kMaxPairPasses * 4, r->stream));
     chk(hipMemsetAsync(r->counters, 0, V * kCounterWords * 4, r->stream));
-    chk(hipMemsetAsync(r->depth_hist, 0, V * kMaxDepthPasses * 1024 * 4, r->stream));
-    chk(hipMemsetAsync(r->pair_hist, 0, V * kMaxPairPasses * 256 * 4, r->stream));
+    chk(hipMemsetAsync(r->depth_hist, 0, V * kHistCopies * kDepthHist * 4, r->stream));
+    chk(hipMemsetAsync(r->pair_hist, 0, V * kHistCopies * kPairHist * 4, r->stream));
     chk(hipStreamSynchronize(r->stream));
   }
   if (e != hipSuccess) {
@@ -827,8 +835,8 @@ int render_frame_scratch(spl_device* dev, const spl_configuration* cfg, spl_scen
     take(&r.sort_status, r.sort_words * kMaxDepthPasses);
     take(&r.bin_status, r.bin_words);
     take(&r.pair_status, r.pair_words * kMaxPairPasses);
-    take(&r.depth_hist, (uint64_t)kMaxDepthPasses * 1024);
-    take(&r.pair_hist, (uint64_t)kMaxPairPasses * 256);
+    take(&r.depth_hist, kHistCopies * kDepthHist);
+    take(&r.pair_hist, kHistCopies * kPairHist);
     take(&r.ranges, tiles);
     zero_bytes = off;
     take(&r.d_uniforms, 1);

@@ -72,7 +72,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
 #pragma unroll
     for (int k = 0; k < DPT; ++k) {
       const uint32_t d = tid * DPT + k;
-      hv[k] = d < (uint32_t)RADIX ? hist[d] : 0u;
+      hv[k] = 0u;
+#pragma unroll
+      for (uint32_t c = 0; c < kHistCopies; ++c) hv[k] += d < (uint32_t)RADIX ? hist[c * a.hist_copy + d] : 0u;
       sum += hv[k];
     }
     uint32_t total;

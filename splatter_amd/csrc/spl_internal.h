@@ -91,7 +91,8 @@ constexpr int kCullThreads = 256, kCullItems = 16;   // 4096 splats per cull / p
 constexpr int kSortThreads = 256, kSortItems = 16;   // 4096 keys per sort tile (the narrow form)
 constexpr int kSortThreadsWide = 512;                // 8192 keys per sort tile
 constexpr int kSortThreadsXL = 1024;                 // 16384 keys per sort tile
-constexpr int kBinThreads = 256, kBinItems = 4;      // 1024 draw ranks per bin tile
+constexpr int kBinThreads = 256, kBinItems = 4;      // 1024 draw ranks per bin tile, 256 in small batches
+constexpr uint32_t kHistCopies = 8;                  // of each view's digit histograms, summed by the sort
 constexpr int kCullTile = kCullThreads * kCullItems;
 
 struct CullLaunch {
@@ -107,7 +108,8 @@ struct CullLaunch {
   uint32_t* tile_prefix; size_t tp_stride;   // [views][cull tiles] exclusive prefix
   uint32_t* status; size_t status_stride;    // [views][cull tiles]
   uint32_t* counters;                        // [views][kCounterWords]
-  uint32_t* hist;                            // one view: [passes << bits] digit histograms; null: not here
+  uint32_t* hist;                            // one view: kHistCopies digit histograms; null: not here
+  size_t hist_copy;                          // words between them
   int bits;
   int grid;
 };
@@ -132,6 +134,7 @@ struct SortPassLaunch {
   uint32_t count_cap;
   int shift;
   const uint32_t* hist; size_t hist_stride;  // this pass's histogram, per view
+  size_t hist_copy;          // words between its kHistCopies copies
   uint32_t* status; size_t status_stride;    // [tiles][radix], per view
   int tile_slot;             // counter slot of this pass's tile counter
   uint32_t* clear_a; size_t clear_a_words; size_t clear_a_stride;
@@ -165,13 +168,14 @@ struct BinLaunch {
   uint32_t* pair_keys;
   uint32_t* pair_vals; size_t pair_stride;
   uint32_t pair_cap;
-  uint32_t* hist; size_t hist_stride;          // [pair passes][256] per view, accumulated
+  uint32_t* hist; size_t hist_stride;          // [kHistCopies][kMaxPairPasses][256] per view, accumulated
   int pair_passes;
   uint64_t* status; size_t status_stride;
   uint32_t* counters;
   // finished bookkeeping of the depth sort, zeroed here (per view)
   uint32_t* clear_a; size_t clear_a_words, clear_a_stride;
   uint32_t* clear_b; size_t clear_b_words, clear_b_stride;
+  int items;                                   // entries a lane: kBinItems or 1
   int grid_x, views;
 };
 

@@ -124,3 +124,29 @@ def test_heavy_tiles(count, logit, width, height, unaligned, blend):
     case.renderer.render_views([case.frame, other], [case.cam] * 2, [case.view] * 2, case.scene)
     got = case.frame.read()
     assert np.array_equal(got[..., [2, 1, 0, 3]] if case.cfg.frame_format == sa.FrameFormat.BGRA8_UNORM else got, img)
+
+
+# Bin tiles of 256 entries up to 2^17 splats in the batch and of 1024 beyond,
+# whose pairs expand 4096 slots at a time: one splat that covers thousands of
+# screen tiles, a tile's pairs just below and above 4096, boxes as wide as the
+# frame
+@pytest.mark.parametrize("count,big,width,height", [(1, 1, 2048, 1024), (256, 1, 1024, 1008), (257, 256, 64, 64),
+                                                    (1024, 1024, 32, 32), (1025, 1024, 48, 32), (5000, 300, 320, 240),
+                                                    ((1 << 17) + 1, 64, 640, 480)])
+@pytest.mark.parametrize("views", [1, 2])
+def test_bin_slots(count, big, width, height, views):
+    say(f"{count} splats, {big} of them large, {width}x{height}, {views} views")
+    rec = Workload("gaussian", count, seed=61).all()
+    rec["center"][:big] *= 0.2
+    rec["scale"][:big] = 1.0     # e, as large as the view
+    rec["alpha"][:big] = -5.0
+    cfg = config(max_splat_count=count, max_views=views, tile_pairs_per_splat=16384 if count < 2000 else 64)
+    case = Case(Workload("gaussian", 0, seed=0), cfg, width, height, sphere_pose(61, radius=5))
+    case.records, case.splats = rec, ob.decode(rec)
+    case.scene = sa.Scene(case.renderer, count)
+    case.scene.load_records(0, rec)
+    others = [sa.Frame(device(), 33, 17) for _ in range(views - 1)]
+    case.renderer.render_views([case.frame] + others, [case.cam] * views, [case.view] * views, case.scene)
+    say(f"  pairs {case.renderer.pair_count()}")
+    _, _, _, oimg = case.oracle()
+    assert image_diff(case.frame.read()[..., [2, 1, 0, 3]], oimg) <= IMAGE_TOL
