@@ -289,8 +289,8 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   // and pay for a tile's own chain (a 1024-lane block ranks four waves a
   // SIMD), large ones for the look-back over many tiles; us, one view on
   // MI355X, depth sort / pair sort in tiles of 4096, 8192 and 16384 keys:
-  //   20k splats   54 / 16    58 / 17    72 / 22
-  //   100k         53 / 33    59 / 32    75 / 38
+  //   20k splats   54 / 16    58 / 17    72 / 22    (1024 keys: 31 / 11)
+  //   100k         51 / 31    59 / 32    75 / 38    (1024 keys: 40 / 34)
   //   1M           67 / 43    67 / 40    79 / 43
   //   1.5M         72 / 44    69 / 40    79 / 44
   //   3M at 4K     93 / 98    84 / 83    91 / 79
@@ -300,14 +300,17 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   };
   const int depth_threads = nv == 1 ? one_view(1u << 19, 1u << 22) : r->sort_threads;
   const int pair_threads = nv == 1 ? one_view(1u << 18, 1u << 21) : r->sort_threads;
-  const auto sort_grid = [&](uint64_t keys, int threads) {
+  const int depth_items = nv == 1 && n <= kSmallSort ? kSortItemsSmall : kSortItems;
+  const int pair_items = nv == 1 && n <= kSmallPairs && r->pair_words >= (size_t)div_up(r->pair_cap, 1024) * 256
+                             ? kSortItemsSmall : kSortItems;
+  const auto sort_grid = [&](uint64_t keys, int threads, int items) {
     const uint32_t per_view = std::max<uint32_t>(1, cus * 4 * kSortThreads / threads / nv);
-    return (int)std::max<uint64_t>(1, std::min<uint64_t>(div_up(keys, (uint64_t)threads * kSortItems), per_view));
+    return (int)std::max<uint64_t>(1, std::min<uint64_t>(div_up(keys, (uint64_t)threads * items), per_view));
   };
   const size_t cap = r->cap;
   const size_t sort_stride = r->sort_words * kMaxDepthPasses;
   const size_t pair_stride_status = r->pair_words * kMaxPairPasses;
-  const size_t sort_used = (size_t)div_up(n, kSortThreads * kSortItems) * radix;
+  const size_t sort_used = (size_t)div_up(n, kSortThreads * depth_items) * radix;
   const size_t cull_used = div_up(n, kCullTile);
   auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], q); };
   // A sorted batch projects on the side stream while the depth sort runs
@@ -417,7 +420,8 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_stride = r->cull_tiles;
     }
     a.threads = depth_threads;
-    a.grid_x = sort_grid(n, depth_threads);
+    a.items = depth_items;
+    a.grid_x = sort_grid(n, depth_threads, depth_items);
     a.views = (int)nv;
     // keys are below 2^30 (0 < clip.z < 1): the last 8-bit pass needs 6 bits
     launch_sort_pass(std::min(bits, 30 - p * bits), a, q);
@@ -479,10 +483,12 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     } else {
       a.clear_a = r->pair_status + (size_t)(p - 1) * r->pair_words;
       a.clear_a_words = r->pair_words;
+      a.clear_a_tile = (uint32_t)(pair_threads * pair_items);
       a.clear_a_stride = pair_stride_status;
     }
     a.threads = pair_threads;
-    a.grid_x = sort_grid(r->pair_cap, pair_threads);
+    a.items = pair_items;
+    a.grid_x = sort_grid(r->pair_cap, pair_threads, pair_items);
     a.views = (int)nv;
     // tile keys are below max_tiles: the last pass takes only their top bits
     launch_sort_pass(std::max(5, std::min(8, tile_bits - 8 * p)), a, q);
@@ -498,6 +504,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.ranges = r->ranges; a.ranges_stride = r->ranges_cap;
     a.clear_a = r->pair_status + (size_t)(Q - 1) * r->pair_words;
     a.clear_a_words = r->pair_words;
+    a.clear_a_tile = (uint32_t)(pair_threads * pair_items);
     a.clear_a_stride = pair_stride_status;
     a.clear_b = r->pair_hist;
     a.clear_b_words = kHistCopies * kPairHist;
@@ -710,9 +717,14 @@ void size_workspace(spl_renderer* r, const spl_configuration* cfg, uint64_t cap,
   r->pair_cap = std::min<uint64_t>(pair_cap, (1ull << 30) - (1ull << 20)) & ~3ull;
   if (r->pair_cap == 0) r->pair_cap = 4;
   r->cull_tiles = div_up(r->cap, kCullTile);
-  r->sort_words = (size_t)div_up(r->cap, kSortThreads * kSortItems) * radix;
+  // tiles of 4096 keys, or as many of 1024 as a small scene has
+  const auto sort_tiles = [](uint64_t keys, uint64_t small) {
+    return (size_t)std::max<uint64_t>(div_up(keys, kSortThreads * kSortItems),
+                                      std::min<uint64_t>(div_up(keys, kSortThreads * kSortItemsSmall), small / 1024));
+  };
+  r->sort_words = sort_tiles(r->cap, kSmallSort) * radix;
   r->bin_words = div_up(r->cap, kBinThreads);
-  r->pair_words = (size_t)div_up(r->pair_cap, kSortThreads * kSortItems) * 256;
+  r->pair_words = sort_tiles(r->pair_cap, 1u << 20) * 256;
 }
 
 }  // namespace

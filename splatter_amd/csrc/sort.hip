@@ -8,7 +8,7 @@
 //    bumped by the lowest peer) carries the rank across the wave's items.
 //    Items are visited in input order, so the pass is stable -- the
 //    reference ranks with LDS atomicAdd (shaders.wgsl:428-429), which is not.
-//  - tiles are TILE = THREADS*ITEMS keys (4096, 8192 or 16384) taken in order from an
+//  - tiles are TILE = THREADS*ITEMS keys (1024 to 16384) taken in order from an
 //    atomic counter by a persistent grid (reference: 1024-key tiles, one
 //    workgroup each, shaders.wgsl:406-420); full tiles skip every per-key
 //    bounds test.
@@ -50,9 +50,10 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & (kWave - 1), w = tid / kWave;
   const uint32_t v = blockIdx.y;
-  if (a.clear_a) clear_words(a.clear_a + v * a.clear_a_stride, a.clear_a_words);
-  if (a.clear_b) clear_words(a.clear_b + v * a.clear_b_stride, a.clear_b_words);
   uint32_t* counters = a.counters + (size_t)v * kCounterWords;
+  if (a.clear_a)
+    clear_words(a.clear_a + v * a.clear_a_stride, used_status(a.clear_a_words, a.clear_a_tile, counters[a.count_slot]));
+  if (a.clear_b) clear_words(a.clear_b + v * a.clear_b_stride, a.clear_b_words);
   const uint32_t* keys_in = a.keys_in + v * a.entry_stride;
   const uint32_t* vals_in = a.vals_in ? a.vals_in + v * a.entry_stride : nullptr;
   uint32_t* keys_out = a.keys_out + v * a.entry_stride;
@@ -271,6 +272,8 @@ void launch_sort_pass_as(const SortPassLaunch& a, hipStream_t s) {
     hipLaunchKernelGGL((k_onesweep_pass<BITS, kSortThreadsXL, kSortItems>), grid, dim3(kSortThreadsXL), 0, s, a);
   else if (a.threads == kSortThreadsWide)
     hipLaunchKernelGGL((k_onesweep_pass<BITS, kSortThreadsWide, kSortItems>), grid, dim3(kSortThreadsWide), 0, s, a);
+  else if (a.items == kSortItemsSmall)
+    hipLaunchKernelGGL((k_onesweep_pass<BITS, kSortThreads, kSortItemsSmall>), grid, dim3(kSortThreads), 0, s, a);
   else
     hipLaunchKernelGGL((k_onesweep_pass<BITS, kSortThreads, kSortItems>), grid, dim3(kSortThreads), 0, s, a);
 }

@@ -191,6 +191,14 @@ __device__ __forceinline__ uint32_t take_ticket(uint32_t* counter, uint32_t num_
   return t;
 }
 
+// Words of a finished sort pass's status to zero: of the capacity's `words`,
+// those of the tiles (`tile` keys, at most 256 digits) that `count` keys had;
+// tile 0: all.
+__device__ __forceinline__ size_t used_status(size_t words, uint32_t tile, uint32_t count) {
+  const size_t used = tile ? ((size_t)count + tile - 1) / tile * 256 : words;
+  return used < words ? used : words;
+}
+
 // Grid-stride zeroing of another stage's finished bookkeeping.
 __device__ __forceinline__ void clear_words(uint32_t* p, size_t n) {
   if (!p) return;

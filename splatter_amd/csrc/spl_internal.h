@@ -89,6 +89,8 @@ constexpr float kShConstants[16] = {
 
 constexpr int kCullThreads = 256, kCullItems = 16;   // 4096 splats per cull / project tile
 constexpr int kSortThreads = 256, kSortItems = 16;   // 4096 keys per sort tile (the narrow form)
+constexpr int kSortItemsSmall = 4;                   // 1024 keys per sort tile: one view of a small scene
+constexpr uint32_t kSmallSort = 1u << 17, kSmallPairs = 1u << 15;  // its splats: depth sort, pair sort
 constexpr int kSortThreadsWide = 512;                // 8192 keys per sort tile
 constexpr int kSortThreadsXL = 1024;                 // 16384 keys per sort tile
 constexpr int kBinThreads = 256, kBinItems = 4;      // 1024 draw ranks per bin tile, 256 in small batches
@@ -139,7 +141,9 @@ struct SortPassLaunch {
   int tile_slot;             // counter slot of this pass's tile counter
   uint32_t* clear_a; size_t clear_a_words; size_t clear_a_stride;
   uint32_t* clear_b; size_t clear_b_words; size_t clear_b_stride;
-  int threads;               // kSortThreads, kSortThreadsWide or kSortThreadsXL lanes, kSortItems keys each
+  uint32_t clear_a_tile;     // keys per tile of the status at clear_a (used_status); 0: clear_a_words it is
+  int threads;               // kSortThreads, kSortThreadsWide or kSortThreadsXL lanes
+  int items;                 // keys a lane: kSortItems, or kSortItemsSmall with kSortThreads
   int grid_x, views;
 };
 
@@ -186,6 +190,7 @@ struct RangesLaunch {
   const Uniforms* uniforms;
   uint2* ranges; size_t ranges_stride;
   uint32_t* clear_a; size_t clear_a_words; size_t clear_a_stride;
+  uint32_t clear_a_tile;     // as in SortPassLaunch
   uint32_t* clear_b; size_t clear_b_words; size_t clear_b_stride;
   int grid_x, views;
 };

@@ -62,9 +62,10 @@ def test_blocks_that_share_a_cull_tile(count, views):
         assert normwise_rel(rec[:, 4:], orec[:, 4:]).max() <= RECORD_TOL
 
 
-# one view sorts depths in 4096-key tiles up to 2^19 splats, in 8192-key tiles
-# up to 2^22 and in 16384-key tiles beyond; pairs change at 2^18 and 2^21
-@pytest.mark.parametrize("count", [1 << 18, (1 << 18) + 1, 1 << 19, (1 << 19) + 1, (1 << 21) + 1, (1 << 22) + 1])
+# one view sorts depths in 1024-key tiles up to 2^17 splats, in 4096-key tiles
+# up to 2^19, in 8192-key tiles up to 2^22 and in 16384-key tiles beyond; pairs
+# change at 2^15, 2^18 and 2^21
+@pytest.mark.parametrize("count", [1000, 1 << 15, (1 << 15) + 1, 1 << 17, (1 << 17) + 1, 1 << 18, (1 << 18) + 1, 1 << 19, (1 << 19) + 1, (1 << 21) + 1, (1 << 22) + 1])
 @pytest.mark.parametrize("bits", [8, 10])
 def test_sort_tile_of_one_view(count, bits):
     say(f"{count} splats, {bits}-bit digits")
