@@ -572,8 +572,10 @@ int spl_frame_read(spl_frame* f, void* host, uint64_t size) {
   const uint64_t need = (uint64_t)f->width * f->height * 4;
   if (size < need) return fail(SPL_ERROR_INVALID_ARGUMENT, "spl_frame_read: buffer too small");
   HIP_TRY(hipSetDevice(f->dev->ordinal));
+  // queued behind the frame: waiting for it first and copying then costs a
+  // round trip to the device more (a 1080p frame into pinned memory)
+  HIP_TRY(hipMemcpyAsync(host, f->pixels, need, hipMemcpyDeviceToHost, f->dev->stream));
   HIP_TRY(hipStreamSynchronize(f->dev->stream));
-  HIP_TRY(hipMemcpy(host, f->pixels, need, hipMemcpyDeviceToHost));
   return SPL_OK;
 }
 

@@ -576,15 +576,19 @@ int enqueue_batch(spl_renderer* r, spl_scene* s, uint32_t nv, spl_frame* const* 
   rc = ensure_tile_work(r, max_tiles);
   if (rc) return rc;
 
-  // stage this batch's uniforms and frame pointers through pinned memory
-  UploadSlot& slot = r->slots[r->next_slot];
-  r->next_slot = (r->next_slot + 1) % kStageSlots;
-  HIP_TRY(hipEventSynchronize(slot.done));
-  std::memcpy(slot.uniforms, u, nv * sizeof(Uniforms));
-  for (uint32_t v = 0; v < nv; ++v) slot.pixels[v] = frames[v]->pixels;
-  HIP_TRY(hipMemcpyAsync(r->d_uniforms, slot.uniforms, nv * sizeof(Uniforms), hipMemcpyHostToDevice, q));
-  HIP_TRY(hipMemcpyAsync(r->d_pixels, slot.pixels, nv * sizeof(uint32_t*), hipMemcpyHostToDevice, q));
-  HIP_TRY(hipEventRecord(slot.done, q));
+  uint32_t* pixels[kMaxViews];
+  for (uint32_t v = 0; v < nv; ++v) pixels[v] = frames[v]->pixels;
+  if (!launch_upload(u, pixels, nv, r->d_uniforms, r->d_pixels, q)) {
+    // stage this batch's uniforms and frame pointers through pinned memory
+    UploadSlot& slot = r->slots[r->next_slot];
+    r->next_slot = (r->next_slot + 1) % kStageSlots;
+    HIP_TRY(hipEventSynchronize(slot.done));
+    std::memcpy(slot.uniforms, u, nv * sizeof(Uniforms));
+    std::memcpy(slot.pixels, pixels, nv * sizeof(uint32_t*));
+    HIP_TRY(hipMemcpyAsync(r->d_uniforms, slot.uniforms, nv * sizeof(Uniforms), hipMemcpyHostToDevice, q));
+    HIP_TRY(hipMemcpyAsync(r->d_pixels, slot.pixels, nv * sizeof(uint32_t*), hipMemcpyHostToDevice, q));
+    HIP_TRY(hipEventRecord(slot.done, q));
+  }
 
   BatchShape b;
   b.scene = s;

@@ -236,6 +236,11 @@ void launch_ranges(const RangesLaunch& a, hipStream_t s);
 void launch_heavy_tiles(const HeavyLaunch& a, hipStream_t s);
 void launch_raster(const RasterLaunch& a, hipStream_t s);
 
+// Writes a batch's uniforms and frame pointers with one kernel that carries
+// them in its arguments; false for more views than those hold.
+bool launch_upload(const Uniforms* u, uint32_t* const* pixels, uint32_t views, Uniforms* d_uniforms,
+                   uint32_t** d_pixels, hipStream_t s);
+
 // spl_render_frame_static: the scratch array's size and the largest scene and
 // frame it takes.
 constexpr uint64_t kStaticScratchBytes = 48ull << 20;

@@ -34,9 +34,49 @@ __global__ __launch_bounds__(256) void k_static_setup(spl::Uniforms u, uint32_t*
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < zero_words; i += stride) zero[i] = 0u;
 }
 
+// A batch's uniforms and frame pointers, by value: one launch, where copies
+// from pinned memory took two blits of 4 us, 13 us apart, before the frame's
+// first kernel, and an event to know when the memory is free again.
+template <int N>
+struct UploadArgs {
+  spl::Uniforms uniforms[N];
+  uint32_t* pixels[N];
+};
+
+template <int N>
+__global__ __launch_bounds__(256) void k_upload(UploadArgs<N> args, spl::Uniforms* d_uniforms, uint32_t** d_pixels,
+                                                uint32_t views) {
+  const uint32_t v = threadIdx.x / 8, lane = threadIdx.x % 8;
+  if (v >= (uint32_t)N || v >= views) return;
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(&args.uniforms[v]);
+  uint32_t* dst = reinterpret_cast<uint32_t*>(&d_uniforms[v]);
+  for (uint32_t i = lane; i < sizeof(spl::Uniforms) / 4; i += 8) dst[i] = src[i];
+  if (lane == 0) d_pixels[v] = args.pixels[v];
+}
+
+template <int N>
+void launch_upload_as(const spl::Uniforms* u, uint32_t* const* pixels, uint32_t views, spl::Uniforms* d_uniforms,
+                      uint32_t** d_pixels, hipStream_t s) {
+  UploadArgs<N> args{};
+  static_assert(sizeof(args) <= 4000, "kernel arguments");
+  for (uint32_t v = 0; v < views; ++v) {
+    args.uniforms[v] = u[v];
+    args.pixels[v] = pixels[v];
+  }
+  hipLaunchKernelGGL((k_upload<N>), dim3(1), dim3(256), 0, s, args, d_uniforms, d_pixels, views);
+}
+
 }  // namespace
 
 namespace spl {
+
+bool launch_upload(const Uniforms* u, uint32_t* const* pixels, uint32_t views, Uniforms* d_uniforms,
+                   uint32_t** d_pixels, hipStream_t s) {
+  if (views == 1) launch_upload_as<1>(u, pixels, views, d_uniforms, d_pixels, s);
+  else if (views <= 8) launch_upload_as<8>(u, pixels, views, d_uniforms, d_pixels, s);
+  else return false;
+  return true;
+}
 
 void launch_static_setup(const Uniforms& u, uint32_t* pixels, Uniforms* d_uniforms, uint32_t** d_pixels,
                          uint32_t* zero, size_t zero_words, hipStream_t s) {
