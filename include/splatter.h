@@ -91,8 +91,9 @@ typedef struct spl_configuration {
     uint32_t tile_pairs_per_splat;        /* capacity of (splat, screen tile) pairs, per max_splat_count */
     uint32_t max_views;                   /* views per batched launch (1..=32); workspace scales with it */
     int32_t use_hip_graphs;               /* replay each batch shape's launch sequence from a hipGraph */
-    uint32_t sort_tile_keys;              /* keys per radix-sort tile: 4096, 8192 or 16384 (256, 512 or
-                                             1024 lanes) */
+    uint32_t sort_tile_keys;              /* keys per radix-sort tile: 4096, 8192 or 16384 (batches of two
+                                             or more views, at least 8192 above 2^22 splats; one view
+                                             goes by the scene's size) */
     uint32_t raster_mode;                 /* 0: each wave's lanes test every entry of its 8x8 quadrant;
                                              1: each lane walks the entries covering its pixel;
                                              2: four lane groups step through the lists of their 4x4

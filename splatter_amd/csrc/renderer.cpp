@@ -70,7 +70,7 @@ struct spl_renderer {
   uint64_t cap = 0;
   uint32_t max_views = 1;
   int depth_bits = 8, depth_passes = 4;
-  int sort_threads = kSortThreads;  // lanes per radix-sort tile
+  int sort_tile = kSortTile;  // keys per radix-sort tile of the batches
   uint64_t pair_cap = 0;
   // per-view sizes (words)
   size_t cull_tiles = 0, sort_words = 0, bin_words = 0, pair_words = 0;
@@ -286,31 +286,36 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   // by the views (which sort side by side, so their look-back chains overlap)
   // A single view picks its tile by the scene's size, whatever the batches
   // use (the autotuner picks the batches' tile).  Small scenes leave CUs idle
-  // and pay for a tile's own chain (a 1024-lane block ranks four waves a
-  // SIMD), large ones for the look-back over many tiles; us, one view on
-  // MI355X, depth sort / pair sort in tiles of 4096, 8192 and 16384 keys:
-  //   20k splats   54 / 16    58 / 17    72 / 22    (1024 keys: 31 / 11)
-  //   100k         51 / 31    59 / 32    75 / 38    (1024 keys: 40 / 34)
-  //   1M           67 / 43    67 / 40    79 / 43
-  //   1.5M         72 / 44    69 / 40    79 / 44
-  //   3M at 4K     93 / 98    84 / 83    91 / 79
-  //   6M          126 / 105  103 / 85   101 / 85
-  const auto one_view = [n](uint64_t narrow, uint64_t wide) {
-    return n <= narrow ? kSortThreads : n <= wide ? kSortThreadsWide : kSortThreadsXL;
+  // and pay for a tile's own chain, large ones for the look-back over many
+  // tiles; us, one view on MI355X, depth sort / pair sort in tiles of 1024,
+  // 4096, 8192 and 16384 keys:
+  //   20k splats   31 / 11    54 / 16     58 / 17    72 / 22
+  //   100k         40 / 34    51 / 31     59 / 32    75 / 38
+  //   1M           77 / 72    55 / 39     58 / 36    79 / 43
+  //   1.5M         96 / 74    61 / 41     60 / 37    79 / 44
+  //   3M at 4K    158 / 187   83 / 90     77 / 82    91 / 79
+  //   6M          232 / 217  116 / 100   107 / 90    98 / 85
+  // (20k and 100k in 4096- and 8192-key tiles: of 256 x 16 and 512 x 16 lanes)
+  const auto one_view = [n](uint64_t small, uint64_t narrow, uint64_t wide) {
+    return n <= small ? kSortTileSmall : n <= narrow ? kSortTile : n <= wide ? 8192 : 16384;
   };
-  const int depth_threads = nv == 1 ? one_view(1u << 19, 1u << 22) : r->sort_threads;
-  const int pair_threads = nv == 1 ? one_view(1u << 18, 1u << 21) : r->sort_threads;
-  const int depth_items = nv == 1 && n <= kSmallSort ? kSortItemsSmall : kSortItems;
-  const int pair_items = nv == 1 && n <= kSmallPairs && r->pair_words >= (size_t)div_up(r->pair_cap, 1024) * 256
-                             ? kSortItemsSmall : kSortItems;
-  const auto sort_grid = [&](uint64_t keys, int threads, int items) {
-    const uint32_t per_view = std::max<uint32_t>(1, cus * 4 * kSortThreads / threads / nv);
-    return (int)std::max<uint64_t>(1, std::min<uint64_t>(div_up(keys, (uint64_t)threads * items), per_view));
+  const bool small_pairs = r->pair_words >= (size_t)div_up(r->pair_cap, kSortTileSmall) * 256;
+  // Batches of large scenes sort in larger tiles than configured: 8 views of
+  // 32M splats, depth sort 5.19, 4.66 and 4.36 ms in 4096-, 8192- and
+  // 16384-key tiles, pair sort 12.4, 11.8 and 12.4.
+  const bool large = n > 1u << 22;
+  const int depth_tile = nv == 1 ? one_view(kSmallSort, 1u << 21, 1u << 22) : large ? 16384 : r->sort_tile;
+  const int pair_tile = nv == 1 ? one_view(small_pairs ? kSmallPairs : 0, 1u << 19, 1u << 21)
+                                : std::max(r->sort_tile, large ? 8192 : 0);
+  const int few_keys = nv == 1 || (uint64_t)n * nv <= 1u << 21;
+  const auto sort_grid = [&](uint64_t keys, int tile) {
+    const uint32_t per_view = std::max<uint32_t>(1, cus * 4 / std::max(1, tile / kSortTile) / nv);
+    return (int)std::max<uint64_t>(1, std::min<uint64_t>(div_up(keys, (uint64_t)tile), per_view));
   };
   const size_t cap = r->cap;
   const size_t sort_stride = r->sort_words * kMaxDepthPasses;
   const size_t pair_stride_status = r->pair_words * kMaxPairPasses;
-  const size_t sort_used = (size_t)div_up(n, kSortThreads * depth_items) * radix;
+  const size_t sort_used = (size_t)div_up(n, depth_tile) * radix;
   const size_t cull_used = div_up(n, kCullTile);
   auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], q); };
   // A sorted batch projects on the side stream while the depth sort runs
@@ -419,9 +424,9 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_words = cull_used;
       a.clear_a_stride = r->cull_tiles;
     }
-    a.threads = depth_threads;
-    a.items = depth_items;
-    a.grid_x = sort_grid(n, depth_threads, depth_items);
+    a.tile_keys = depth_tile;
+    a.few = few_keys;
+    a.grid_x = sort_grid(n, depth_tile);
     a.views = (int)nv;
     // keys are below 2^30 (0 < clip.z < 1): the last 8-bit pass needs 6 bits
     launch_sort_pass(std::min(bits, 30 - p * bits), a, q);
@@ -483,12 +488,12 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     } else {
       a.clear_a = r->pair_status + (size_t)(p - 1) * r->pair_words;
       a.clear_a_words = r->pair_words;
-      a.clear_a_tile = (uint32_t)(pair_threads * pair_items);
+      a.clear_a_tile = (uint32_t)pair_tile;
       a.clear_a_stride = pair_stride_status;
     }
-    a.threads = pair_threads;
-    a.items = pair_items;
-    a.grid_x = sort_grid(r->pair_cap, pair_threads, pair_items);
+    a.tile_keys = pair_tile;
+    a.few = few_keys;
+    a.grid_x = sort_grid(r->pair_cap, pair_tile);
     a.views = (int)nv;
     // tile keys are below max_tiles: the last pass takes only their top bits
     launch_sort_pass(std::max(5, std::min(8, tile_bits - 8 * p)), a, q);
@@ -504,7 +509,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.ranges = r->ranges; a.ranges_stride = r->ranges_cap;
     a.clear_a = r->pair_status + (size_t)(Q - 1) * r->pair_words;
     a.clear_a_words = r->pair_words;
-    a.clear_a_tile = (uint32_t)(pair_threads * pair_items);
+    a.clear_a_tile = (uint32_t)pair_tile;
     a.clear_a_stride = pair_stride_status;
     a.clear_b = r->pair_hist;
     a.clear_b_words = kHistCopies * kPairHist;
@@ -713,8 +718,7 @@ void size_workspace(spl_renderer* r, const spl_configuration* cfg, uint64_t cap,
   r->depth_passes = (30 + r->depth_bits - 1) / r->depth_bits;
   if (r->cfg.sort_tile_keys == 0) r->cfg.sort_tile_keys = 4096;
   if (r->cfg.raster_batch == 0) r->cfg.raster_batch = 128;
-  r->sort_threads = r->cfg.sort_tile_keys == 16384 ? kSortThreadsXL
-                    : r->cfg.sort_tile_keys == 8192 ? kSortThreadsWide : kSortThreads;
+  r->sort_tile = (int)r->cfg.sort_tile_keys;
   const int radix = 1 << r->depth_bits;
   // a multiple of 4: the tile-range pass reads the pair keys as uint4
   if (pair_cap == 0) pair_cap = r->cap * (uint64_t)r->cfg.tile_pairs_per_splat;
@@ -723,8 +727,8 @@ void size_workspace(spl_renderer* r, const spl_configuration* cfg, uint64_t cap,
   r->cull_tiles = div_up(r->cap, kCullTile);
   // tiles of 4096 keys, or as many of 1024 as a small scene has
   const auto sort_tiles = [](uint64_t keys, uint64_t small) {
-    return (size_t)std::max<uint64_t>(div_up(keys, kSortThreads * kSortItems),
-                                      std::min<uint64_t>(div_up(keys, kSortThreads * kSortItemsSmall), small / 1024));
+    return (size_t)std::max<uint64_t>(div_up(keys, kSortTile),
+                                      std::min<uint64_t>(div_up(keys, kSortTileSmall), small / kSortTileSmall));
   };
   r->sort_words = sort_tiles(r->cap, kSmallSort) * radix;
   r->bin_words = div_up(r->cap, kBinThreads);

@@ -265,17 +265,28 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
   }
 }
 
+// Lanes and keys a lane of each tile size.  Few keys in all (`few`): eight or
+// four keys a lane shorten a tile's chain of rankings; one view, depth sort /
+// pair sort in us: 1M splats in 4096-key tiles of 512 x 8 lanes 55 / 39, of
+// 256 x 16 66 / 43; in 8192-key tiles of 1024 x 8 58 / 36, of 512 x 16
+// 66 / 40; five views of 300k in 4096-key tiles 48 / 31 against 59 / 35.  With
+// many, sixteen keys a lane keep more tiles on a CU: 8 views of 32M a pass of
+// 63.3 ms with 256 x 16, 65.3 with 512 x 8.
 template <int BITS>
 void launch_sort_pass_as(const SortPassLaunch& a, hipStream_t s) {
   const dim3 grid(a.grid_x, a.views);
-  if (a.threads == kSortThreadsXL)
-    hipLaunchKernelGGL((k_onesweep_pass<BITS, kSortThreadsXL, kSortItems>), grid, dim3(kSortThreadsXL), 0, s, a);
-  else if (a.threads == kSortThreadsWide)
-    hipLaunchKernelGGL((k_onesweep_pass<BITS, kSortThreadsWide, kSortItems>), grid, dim3(kSortThreadsWide), 0, s, a);
-  else if (a.items == kSortItemsSmall)
-    hipLaunchKernelGGL((k_onesweep_pass<BITS, kSortThreads, kSortItemsSmall>), grid, dim3(kSortThreads), 0, s, a);
+  if (a.tile_keys == 16384)
+    hipLaunchKernelGGL((k_onesweep_pass<BITS, 1024, 16>), grid, dim3(1024), 0, s, a);
+  else if (a.tile_keys == 8192 && a.few)
+    hipLaunchKernelGGL((k_onesweep_pass<BITS, 1024, 8>), grid, dim3(1024), 0, s, a);
+  else if (a.tile_keys == 8192)
+    hipLaunchKernelGGL((k_onesweep_pass<BITS, 512, 16>), grid, dim3(512), 0, s, a);
+  else if (a.tile_keys == kSortTileSmall)
+    hipLaunchKernelGGL((k_onesweep_pass<BITS, 256, 4>), grid, dim3(256), 0, s, a);
+  else if (a.few)
+    hipLaunchKernelGGL((k_onesweep_pass<BITS, 512, 8>), grid, dim3(512), 0, s, a);
   else
-    hipLaunchKernelGGL((k_onesweep_pass<BITS, kSortThreads, kSortItems>), grid, dim3(kSortThreads), 0, s, a);
+    hipLaunchKernelGGL((k_onesweep_pass<BITS, 256, 16>), grid, dim3(256), 0, s, a);
 }
 
 // bits: the digit width of this pass, 5..8 or 10.  A pass over the top

@@ -88,11 +88,9 @@ constexpr float kShConstants[16] = {
 };
 
 constexpr int kCullThreads = 256, kCullItems = 16;   // 4096 splats per cull / project tile
-constexpr int kSortThreads = 256, kSortItems = 16;   // 4096 keys per sort tile (the narrow form)
-constexpr int kSortItemsSmall = 4;                   // 1024 keys per sort tile: one view of a small scene
-constexpr uint32_t kSmallSort = 1u << 17, kSmallPairs = 1u << 15;  // its splats: depth sort, pair sort
-constexpr int kSortThreadsWide = 512;                // 8192 keys per sort tile
-constexpr int kSortThreadsXL = 1024;                 // 16384 keys per sort tile
+constexpr int kSortTile = 4096;                      // keys per sort tile: 4096, 8192 or 16384,
+constexpr int kSortTileSmall = 1024;                 // or these, for one view of a small scene:
+constexpr uint32_t kSmallSort = 1u << 17, kSmallPairs = 1u << 15;  // its splats (depth sort, pair sort)
 constexpr int kBinThreads = 256, kBinItems = 4;      // 1024 draw ranks per bin tile, 256 in small batches
 constexpr uint32_t kHistCopies = 8;                  // of each view's digit histograms, summed by the sort
 constexpr int kCullTile = kCullThreads * kCullItems;
@@ -142,8 +140,8 @@ struct SortPassLaunch {
   uint32_t* clear_a; size_t clear_a_words; size_t clear_a_stride;
   uint32_t* clear_b; size_t clear_b_words; size_t clear_b_stride;
   uint32_t clear_a_tile;     // keys per tile of the status at clear_a (used_status); 0: clear_a_words it is
-  int threads;               // kSortThreads, kSortThreadsWide or kSortThreadsXL lanes
-  int items;                 // keys a lane: kSortItems, or kSortItemsSmall with kSortThreads
+  int tile_keys;             // 1024, 4096, 8192 or 16384
+  int few;                   // few keys in all: more lanes with fewer keys each
   int grid_x, views;
 };
 
