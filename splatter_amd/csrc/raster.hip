@@ -348,7 +348,7 @@ __global__ __launch_bounds__(256) void k_tile_ranges(RangesLaunch a) {
     clear_words(a.clear_a + v * a.clear_a_stride,
                 used_status(a.clear_a_words, a.clear_a_tile, a.counters[(size_t)v * kCounterWords + kPairs]));
   if (a.clear_b) clear_words(a.clear_b + v * a.clear_b_stride, a.clear_b_words);
-  if (blockIdx.x == 0 && v == 0 && threadIdx.x <= kHeavyClasses) a.counters[kHeavyAll + threadIdx.x] = 0u;
+  if (blockIdx.x == 0 && v == 0 && threadIdx.x <= kHeavyClasses + 1) a.counters[kHeavyAll + threadIdx.x] = 0u;
   const uint32_t* keys = a.pair_keys + v * a.pair_stride;  // 16-byte aligned: pair_stride % 4 == 0
   uint2* ranges = a.ranges + v * a.ranges_stride;
   const uint32_t tiles = a.uniforms[v].tiles_x * a.uniforms[v].tiles_y;
@@ -398,7 +398,16 @@ __global__ __launch_bounds__(256) void k_heavy_tiles(HeavyLaunch a) {
   uint2* range = a.ranges + v * a.ranges_stride + t;
   const uint2 r = *range;
   const uint32_t len = r.y - r.x;
-  if (len < thr) return;
+  if (len < thr) {
+    // a long tile among the ordinary ones starts ahead of them
+    const uint32_t mine = min(a.counters[(size_t)v * kCounterWords + kPairs], a.pair_cap);
+    if (len < max(thr / 4u, 2u * (mine / T))) return;
+    const uint32_t at = atomicAdd(&a.counters[kLongTiles], 1u);
+    if (at >= a.long_cap) return;
+    a.list[kHeavyClasses * kHeavyCap + at] = (v << 24) | t;
+    range->x = r.x | kHeavyFlag;
+    return;
+  }
   const uint32_t times = len / thr;
   const uint32_t c = times >= 16u ? 3u : times >= 4u ? 2u : times >= 2u ? 1u : 0u;
   uint32_t* const all = a.counters;  // one set of lists for all views, counted in view 0's block
@@ -442,8 +451,8 @@ __global__ __launch_bounds__(256, MODE == 3 ? (B == 128 ? (F32 ? 6 : 7) : 5) : 1
   __shared__ __align__(16) uint8_t s_sub[SUBS ? 4 : 1][SUBS ? 4 : 1][SUBS ? B : 4];  // mode 2: per 4x4 sub-block
 
   // Block -> (view, tile).  First eight blocks for each heavy tile, longest
-  // class first, then each view's tiles in a slot range of slots_per_view
-  // blocks.  Blocks are dealt round-robin to the 8 XCDs, and the XCDs take
+  // class first, then one for each long tile, then each view's tiles in a slot
+  // range of slots_per_view blocks.  Blocks are dealt round-robin to the 8 XCDs, and the XCDs take
   // runs of kXcdRun neighbouring tiles in turn (kXcdRun has why).
   uint32_t b = blockIdx.x;
   const uint32_t heavy = min(a.counters[kHeavyAll], a.heavy_cap), heavy_blocks = 8u * ((heavy + 7u) & ~7u);
@@ -463,11 +472,22 @@ __global__ __launch_bounds__(256, MODE == 3 ? (B == 128 ? (F32 ? 6 : 7) : 5) : 1
     return;
   }
   b -= heavy_blocks;
-  const uint32_t v = b / a.slots_per_view;
-  if (v >= (uint32_t)a.views) return;
-  const uint32_t slot = b % a.slots_per_view;
-  const uint32_t tile = ((slot >> 3) / kXcdRun * 8u + (slot & 7u)) * kXcdRun + (slot >> 3) % kXcdRun;
-  if (tile >= a.uniforms[v].tiles_x * a.uniforms[v].tiles_y) return;
+  uint32_t v, tile;
+  const uint32_t longs = min(a.counters[kLongTiles], a.long_cap), long_blocks = (longs + 7u) & ~7u;
+  const bool listed = b < long_blocks;
+  if (listed) {
+    if (b >= longs) return;
+    const uint32_t vt = a.heavy[kHeavyClasses * kHeavyCap + b];
+    v = vt >> 24;
+    tile = vt & 0xFFFFFFu;
+  } else {
+    b -= long_blocks;
+    v = b / a.slots_per_view;
+    if (v >= (uint32_t)a.views) return;
+    const uint32_t slot = b % a.slots_per_view;
+    tile = ((slot >> 3) / kXcdRun * 8u + (slot & 7u)) * kXcdRun + (slot >> 3) % kXcdRun;
+    if (tile >= a.uniforms[v].tiles_x * a.uniforms[v].tiles_y) return;
+  }
   const Uniforms& u = a.uniforms[v];
   const uint2* ranges = a.ranges + v * a.ranges_stride;
   const uint32_t* pair_vals = a.pair_vals + v * a.pair_stride;
@@ -483,8 +503,9 @@ __global__ __launch_bounds__(256, MODE == 3 ? (B == 128 ? (F32 ? 6 : 7) : 5) : 1
   const uint32_t W = u.image_size[0], H = u.image_size[1];
   const bool inside = px < W && py < H;
   // (the ranges are cleared for the next frame by its pair sort)
-  const uint2 range = ranges[tile];
-  if (range.x & kHeavyFlag) return;  // has blocks of its own
+  uint2 range = ranges[tile];
+  if (listed) range.x &= ~kHeavyFlag;
+  else if (range.x & kHeavyFlag) return;  // has blocks of its own
 
   const PixelMap pm = pixel_map(u);
   const float pxf = (float)px, pyf = (float)py;

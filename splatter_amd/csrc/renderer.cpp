@@ -524,6 +524,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   // 1210 against 1277 us a frame, 1M 561 against 584).
   const uint32_t raster_batch = nv == 1 ? 128u : cfg.raster_batch;
   const uint32_t heavy_cap = std::min<uint32_t>(kHeavyCap, nv * b.max_tiles);
+  const uint32_t long_cap = std::min<uint32_t>(kLongCap, nv * b.max_tiles);
   {
     HeavyLaunch a{};
     a.ranges = r->ranges; a.ranges_stride = r->ranges_cap;
@@ -532,6 +533,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.pair_cap = (uint32_t)r->pair_cap;
     a.list = r->heavy;
     a.heavy_cap = heavy_cap;
+    a.long_cap = long_cap;
     a.tile_work = b.tile_stats ? r->tile_work : nullptr;
     a.max_tiles = b.max_tiles;
     a.views = (int)nv;
@@ -555,7 +557,8 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.heavy = r->heavy;
     a.slots_per_view = slots;
     a.heavy_cap = heavy_cap;
-    a.grid_x = (int)(8 * div_up(heavy_cap, 8) * 8 + nv * slots);
+    a.long_cap = long_cap;
+    a.grid_x = (int)(8 * div_up(heavy_cap, 8) * 8 + div_up(long_cap, 8) * 8 + nv * slots);
     a.views = (int)nv;
     launch_raster(a, q);
   }
@@ -780,7 +783,7 @@ int renderer_create(spl_device* dev, const spl_configuration* cfg, bool own_stre
   chk(alloc(&r->counters, V * kCounterWords));
   chk(alloc(&r->depth_hist, V * kHistCopies * kDepthHist));
   chk(alloc(&r->pair_hist, V * kHistCopies * kPairHist));
-  chk(alloc(&r->heavy, (size_t)kHeavyClasses * kHeavyCap));
+  chk(alloc(&r->heavy, (size_t)kHeavyClasses * kHeavyCap + kLongCap));
   chk(alloc(&r->vis, r->cap));
   chk(alloc(&r->d_uniforms, V));
   chk(alloc(&r->d_pixels, V));
@@ -870,7 +873,7 @@ int render_frame_scratch(spl_device* dev, const spl_configuration* cfg, spl_scen
     take(&r.compact_idx, r.cap);
     take(&r.records, r.cap * kRecordFloat4);
     take(&r.boxes, r.cap);
-    take(&r.heavy, (uint64_t)kHeavyClasses * kHeavyCap);
+    take(&r.heavy, (uint64_t)kHeavyClasses * kHeavyCap + kLongCap);
     for (int i = 0; i < 2; ++i) {
       take(&r.pair_keys[i], r.pair_cap);
       take(&r.pair_vals[i], r.pair_cap);

@@ -52,6 +52,7 @@ enum CounterSlot : int {
   kScatterError = 35,
   kHeavyAll = 36,   // view 0's block: tiles that k_heavy_tiles found heavy
   kHeavyTiles = 37, // .. + kHeavyClasses - 1: tiles in each of its lists
+  kLongTiles = 41,  // view 0's block: tiles that start first among the ordinary ones
   kCounterWords = 64
 };
 
@@ -65,6 +66,9 @@ enum CounterSlot : int {
 // 525, 598; 1.5M at VGA 462, 455, 467, 465; five views of 300k 575, 535, 537,
 // 665 (at 1/2500 they are too many for the eightfold reading to pay).
 constexpr uint32_t kHeavyShare = 1000, kHeavyMin = 512, kHeavyCap = 1000;
+// Of the others, those of a quarter of that and twice the view's mean list
+// start first (kLongCap of them at most).
+constexpr uint32_t kLongCap = 2048;
 constexpr int kHeavyClasses = 4;
 constexpr uint32_t kHeavyFlag = 0x80000000u;  // in a tile range's start (starts are below 2^30)
 
@@ -198,7 +202,8 @@ struct HeavyLaunch {
   const Uniforms* uniforms;
   uint32_t* counters;
   uint32_t pair_cap;
-  uint32_t* list;                            // kHeavyClasses lists of kHeavyCap: view << 24 | tile
+  uint32_t* list;                            // kHeavyClasses lists of kHeavyCap, one of kLongCap: view << 24 | tile
+  uint32_t long_cap;                         // most of those listed: kLongCap, or all tiles
   uint32_t heavy_cap;                        // most tiles listed: kHeavyCap, or all tiles
   uint2* tile_work;                          // optional, view 0, as in RasterLaunch
   uint32_t max_tiles;
@@ -207,7 +212,7 @@ struct HeavyLaunch {
 
 struct RasterLaunch {
   const uint32_t* heavy;     // k_heavy_tiles' lists
-  uint32_t heavy_cap;
+  uint32_t heavy_cap, long_cap;
   uint32_t slots_per_view;   // multiple of 8 * kXcdRun, >= the largest view's tile count
   const uint32_t* pair_vals; size_t pair_stride;
   const float4* records; size_t rec_stride;

@@ -151,3 +151,26 @@ def test_bin_slots(count, big, width, height, views):
     say(f"  pairs {case.renderer.pair_count()}")
     _, _, _, oimg = case.oracle()
     assert image_diff(case.frame.read()[..., [2, 1, 0, 3]], oimg) <= IMAGE_TOL
+
+
+# ordinary tiles with at least 128 pairs (a quarter of the heavy threshold) and
+# twice the view's mean start first, one block each, in single views and batches
+@pytest.mark.parametrize("count,views", [(6000, 1), (6000, 3), (60_000, 2)])
+def test_long_tiles(count, views):
+    say(f"{count} splats, {views} views")
+    case = Case(Workload("gaussian", count, seed=71), config(max_views=views, tile_pairs_per_splat=16), 500, 300,
+                sphere_pose(71, radius=9))
+    case.renderer.enable_tile_stats(True)
+    others = [sa.Frame(device(), 300 - 40 * i, 200) for i in range(views - 1)]
+    case.renderer.render_views([case.frame] + others, [case.cam] * views, [case.view] * views, case.scene)
+    lens = case.renderer.tile_stats()[:, 0].astype(np.int64)
+    few = max(512, lens.sum() // 1000)
+    longs = np.count_nonzero((lens >= max(few // 4, 2 * (lens.sum() // len(lens)))) & (lens < few))
+    say(f"  mean list {lens.mean():.0f}, max {lens.max()}, long tiles {longs}")
+    assert longs > 0
+    _, _, _, oimg = case.oracle()
+    assert image_diff(case.frame.read()[..., [2, 1, 0, 3]], oimg) <= IMAGE_TOL
+    for f in others:  # each view of the batch equals its own frame
+        got = f.read()
+        case.renderer.render_frame(f, case.cam, case.view, case.scene)
+        assert np.array_equal(f.read(), got)
