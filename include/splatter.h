@@ -183,7 +183,7 @@ int spl_render_views(spl_renderer* renderer, spl_scene* scene, uint32_t view_cou
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under stream capture, tight serving loops, harnesses that
  * forbid hipMalloc).  spl_render_frame for one view with no renderer: the
- * whole workspace is a fixed 48 MiB scratch array that the library holds on
+ * whole workspace is a fixed 52 MiB scratch array that the library holds on
  * each device it runs on (looked up once, when the device opens), so the
  * call allocates nothing.  Scenes up to 131072 splats and frames up to
  * 3840 x 2160; larger ones fail with SPL_ERROR_CAPACITY.  config is checked

@@ -246,7 +246,7 @@ bool launch_upload(const Uniforms* u, uint32_t* const* pixels, uint32_t views, U
 
 // spl_render_frame_static: the scratch array's size and the largest scene and
 // frame it takes.
-constexpr uint64_t kStaticScratchBytes = 48ull << 20;
+constexpr uint64_t kStaticScratchBytes = 52ull << 20;
 constexpr uint32_t kStaticMaxSplats = 1u << 17;
 constexpr uint32_t kStaticMaxWidth = 3840, kStaticMaxHeight = 2160;
 // Writes the frame's uniforms and pixel pointer and zeroes `zero_words`
