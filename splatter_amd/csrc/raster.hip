@@ -423,7 +423,7 @@ void launch_heavy_tiles(const HeavyLaunch& a, hipStream_t s) {
 }
 
 // One 256-lane block per 16x16 tile; wave w owns the 8x8 quadrant
-// (w & 1, w >> 1), one lane per pixel.  Entries arrive 256 at a time in draw
+// (w & 1, w >> 1), one lane per pixel.  Entries arrive B at a time in draw
 // order: every lane gathers one record and stores the prepared entry (inverse
 // affine map, translation, coverage half-extent, colour, pixel box) in LDS,
 // while the next batch is already being fetched into registers.  Each wave
