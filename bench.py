@@ -175,16 +175,16 @@ def sort_stress(sa, dev, log, n: int = 32_000_000, width: int = 3840, height: in
     """The depth sort on the stress workload: 32M splats in 16 tight
     clusters (sigma 0.05, dense and tie-heavy f32 depths), 8 orbit views at
     3840x2160 in one batch.  Per-frame stage times from HIP events around
-    every stage of 4 batches, for the two sort shapes the tuner weighs
-    (10-bit digits in 16384-key tiles, 8-bit digits in 4096-key tiles);
+    every stage of 4 batches, for 10-bit and 8-bit digits, both in the tiles
+    that batches of a scene this large take whatever is configured (the
+    result names them);
     Gkeys/s = visible entries / depth-sort time, GB/s = 16 B x passes x
     visible / depth-sort time (key and value read and written per pass)."""
     from splatter_amd.synth import Workload, orbit_poses
     t0 = time.perf_counter()
-    shapes = [(10, 16384), (8, 4096)]
-    rs = [sa.Renderer(dev, sa.Configuration(spherical_harmonics_order=3, max_splat_count=n, max_views=views,
-                                            tile_pairs_per_splat=8, radix_bits_per_digit=b, sort_tile_keys=t))
-          for b, t in shapes]
+    cfgs = [sa.Configuration(spherical_harmonics_order=3, max_splat_count=n, max_views=views,
+                             tile_pairs_per_splat=8, radix_bits_per_digit=b) for b in (10, 8)]
+    rs = [sa.Renderer(dev, cfg) for cfg in cfgs]
     scene = sa.Scene(rs[0], n)
     for first, rec in Workload("tight", n, seed=4).chunks():
         scene.load_records(first, rec)
@@ -194,7 +194,9 @@ def sort_stress(sa, dev, log, n: int = 32_000_000, width: int = 3840, height: in
     frames = [sa.Frame(dev, width, height) for _ in range(views)]
     out = {"workload": f"{n // 1_000_000}M splats in 16 tight clusters (sigma 0.05), {width}x{height}, "
                        f"{views} views per batch"}
-    for (bits, tile), r in zip(shapes, rs):
+    for cfg, r in zip(cfgs, rs):
+        bits = cfg.radix_bits_per_digit
+        tile, pair_tile = sa.sort_tiles(cfg, n, views)
         r.render_views(frames, [p[0] for p in poses], [p[1] for p in poses], scene)
         r.enable_timing(True)
         for _ in range(4):
@@ -214,7 +216,8 @@ def sort_stress(sa, dev, log, n: int = 32_000_000, width: int = 3840, height: in
         out[f"r{bits}_t{tile}"] = {"visible_per_view": int(V), "depth_sort_ms": round(sort_ms, 4),
                                    "gkeys_per_s": round(V / (sort_ms * 1e-3) / 1e9, 2), "passes": P,
                                    "GB/s": round(gbs, 1), "frac_of_8TBs": round(gbs / HBM_PEAK_GBS, 4),
-                                   "pair_sort_ms": round(pair_ms, 4)}
+                                   "pair_sort_ms": round(pair_ms, 4), "depth_tile_keys": tile,
+                                   "pair_tile_keys": pair_tile}
         log(f"sort stress r{bits} t{tile}: {out[f'r{bits}_t{tile}']}")
     for o in frames + [scene] + rs:
         o.close()
@@ -436,14 +439,14 @@ def main() -> int:
     log(f"scene: {args.splats} splats generated+uploaded in {time.perf_counter() - t0:.1f}s")
     poses = orbit_poses(256)
     if args.tune_only:
-        # radix digit width x sort tile (block shape) at this batch width,
+        # radix digit width x sort tile at this batch width,
         # each candidate timed on the same resident scene over the whole
         # orbit, as the timed steps are (the poses differ in cost, so part
         # of the orbit is a different workload)
         pipe[0].close()
         res = at.autotune_staged(sa, dev, cfg, lambda _r: scene, poses, W, H, V_PER,
                                  steps=max(1, len(poses) // V_PER), log=log,
-                                 in_flight=max(1, args.in_flight))
+                                 in_flight=max(1, args.in_flight), splats=args.splats)
         print(json.dumps(res.to_json()), flush=True)
         return 0
     frames = [sa.Frame(dev, W, H) for _ in range(V_PER)]
@@ -608,7 +611,8 @@ def main() -> int:
                                f"256-pose orbit, {V_PER} views per batch",
                    "splats": args.splats, "width": W, "height": H, "views_per_batch": V_PER,
                    "radix_bits_per_digit": cfg.radix_bits_per_digit, "sort_tile_keys": cfg.sort_tile_keys,
-                   "raster_batch": cfg.raster_batch, "raster_longest_first": cfg.raster_longest_first,
+                   "sort_tiles_run": dict(zip(("depth", "pairs"), sa.sort_tiles(cfg, args.splats, V_PER))),
+                   "raster_batch": cfg.raster_batch,
                    "raster_mode": cfg.raster_mode, "batches_in_flight": in_flight,
                    "autotune": tuned.to_json() if tuned else None},
         "plain_frames_per_s": round(plain_fps, 2),

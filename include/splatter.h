@@ -91,9 +91,11 @@ typedef struct spl_configuration {
     uint32_t tile_pairs_per_splat;        /* capacity of (splat, screen tile) pairs, per max_splat_count */
     uint32_t max_views;                   /* views per batched launch (1..=32); workspace scales with it */
     int32_t use_hip_graphs;               /* replay each batch shape's launch sequence from a hipGraph */
-    uint32_t sort_tile_keys;              /* keys per radix-sort tile: 4096, 8192 or 16384 (batches of two
-                                             or more views, at least 8192 above 2^22 splats; one view
-                                             goes by the scene's size) */
+    uint32_t sort_tile_keys;              /* keys per radix-sort tile of batches of two or more views:
+                                             4096, 8192 or 16384.  Of a scene above 2^22 splats they sort
+                                             depths in 16384-key tiles and pairs in at least 8192-key
+                                             ones; one view goes by the scene, whatever is set here
+                                             (spl_debug_sort_tiles tells) */
     uint32_t raster_mode;                 /* 0: each wave's lanes test every entry of its 8x8 quadrant;
                                              1: each lane walks the entries covering its pixel;
                                              2: four lane groups step through the lists of their 4x4
@@ -296,6 +298,12 @@ int spl_debug_read_tile_stats(spl_renderer* renderer, uint32_t* out, uint64_t ca
  * launches rather than graph replays. */
 int spl_debug_enable_timing(spl_renderer* renderer, int enable);
 int spl_debug_stage_times(spl_renderer* renderer, float* ms, uint32_t capacity);
+/* Keys per radix-sort tile that a renderer of `configuration` takes for the
+ * depth sort and for the pair sort of a batch of `views` views of a scene of
+ * `splats` splats, so that a report or a tuner can name what runs.  Needs no
+ * device. */
+int spl_debug_sort_tiles(const spl_configuration* configuration, uint64_t splats, uint32_t views,
+                         uint32_t* depth_tile_keys, uint32_t* pair_tile_keys);
 
 #ifdef __cplusplus
 }

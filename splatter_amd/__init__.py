@@ -30,7 +30,7 @@ from ._lib import (SplConfiguration, SplRequestInfo, SplServerConfiguration, Spl
 
 __all__ = [
     "DepthSorting", "FrameFormat", "BlendMode", "Configuration", "Device", "Renderer",
-    "Scene", "Frame", "Server", "SplatterError", "SERIALIZED_SPLAT_DTYPE",
+    "Scene", "Frame", "Server", "SplatterError", "SERIALIZED_SPLAT_DTYPE", "sort_tiles",
 ]
 
 
@@ -70,7 +70,7 @@ class Configuration:
     tile_pairs_per_splat: int = 4
     max_views: int = 1
     use_hip_graphs: bool = True
-    sort_tile_keys: int = 4096
+    sort_tile_keys: int = 4096       # of batches; large scenes and one view have rules of their own (sort_tiles)
     raster_mode: int = 3             # per-lane walk over coverage masks (every mode renders the same image)
     raster_batch: int = 128          # batches of two or more views; one view rasters with 128
     raster_longest_first: int = 0    # no effect: the longest tiles always start first
@@ -97,6 +97,15 @@ class Configuration:
         c.raster_batch = int(self.raster_batch)
         c.raster_longest_first = int(self.raster_longest_first)
         return c
+
+
+def sort_tiles(config: Configuration, splats: int, views: int) -> tuple[int, int]:
+    """Keys per radix-sort tile of the depth sort and of the pair sort that a
+    batch of `views` views of a scene of `splats` splats runs with."""
+    depth, pairs = C.c_uint32(), C.c_uint32()
+    c = config.to_c()
+    check(lib().spl_debug_sort_tiles(C.byref(c), splats, views, C.byref(depth), C.byref(pairs)))
+    return depth.value, pairs.value
 
 
 # scene.rs:17-24 SerializedSplat, 248 bytes

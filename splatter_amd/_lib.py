@@ -134,6 +134,8 @@ SIGNATURES = [
     ("spl_debug_read_tile_stats", C.c_int, [_P, _P, C.c_uint64, C.POINTER(C.c_uint64)]),
     ("spl_debug_enable_timing", C.c_int, [_P, C.c_int]),
     ("spl_debug_stage_times", C.c_int, [_P, _F16, C.c_uint32]),
+    ("spl_debug_sort_tiles", C.c_int, [C.POINTER(SplConfiguration), C.c_uint64, C.c_uint32, C.POINTER(C.c_uint32),
+                                       C.POINTER(C.c_uint32)]),
 ]
 
 _lib = None

@@ -1,7 +1,7 @@
 """Autotuner for the batched form: picks the radix digit width, the radix-sort
-tile (keys per tile, i.e. the sort block's lane count), the rasteriser's
-batch (entries a tile block stages per round), walk (entry-major, per-pixel,
-per 4x4 sub-block or per-lane over coverage masks) and tile order, and the batch width (views per launch sequence)
+tile (keys per tile), the rasteriser's batch (entries a tile block stages per
+round) and walk (entry-major, per-pixel, per 4x4 sub-block or per-lane over
+coverage masks), and the batch width (views per launch sequence)
 for one scene, resolution and pose set by timing the candidates on the
 device, and can keep the answer in a JSON cache.
 
@@ -22,7 +22,6 @@ RADIX_BITS = (8, 10)
 SORT_TILE_KEYS = (4096, 8192, 16384)
 RASTER_MODE = (0, 1, 2, 3)
 RASTER_BATCH = (128, 256)
-RASTER_LONGEST_FIRST = (0, 1)
 BATCH_VIEWS = (8, 16, 32)
 
 
@@ -33,7 +32,7 @@ class Candidate:
     max_views: int
     raster_mode: int = 0
     raster_batch: int = 128
-    raster_longest_first: int = 0
+    raster_longest_first: int = 0  # no effect on a render, so not searched; kept for cached answers
 
     def key(self) -> str:
         return (f"r{self.radix_bits_per_digit}-t{self.sort_tile_keys}-b{self.raster_batch}-m{self.raster_mode}"
@@ -73,6 +72,30 @@ def candidates(radix_bits=RADIX_BITS, sort_tile_keys=SORT_TILE_KEYS, batch_views
             itertools.product(radix_bits, sort_tile_keys, batch_views, raster_mode)]
 
 
+def configured(base, cand: Candidate):
+    """A copy of the base configuration with the candidate's settings."""
+    cfg = type(base)(**{k: getattr(base, k) for k in base.__dataclass_fields__})
+    TuneResult(cand, 0.0).apply(cfg)
+    return cfg
+
+
+def distinct(sa, base, cands, splats: int):
+    """The candidates without those that would run the launches of an earlier
+    one on a scene of `splats` splats: timed, they would differ by noise, and
+    noise would decide between them.  Large scenes override the sort tile,
+    and one view takes neither the sort tile nor the raster's batch."""
+    seen, out = set(), []
+    for c in cands:
+        cfg = configured(base, c)
+        cfg.max_splat_count = max(cfg.max_splat_count, splats)
+        form = (c.radix_bits_per_digit, *sa.sort_tiles(cfg, splats, c.max_views), c.max_views, c.raster_mode,
+                c.raster_batch if c.max_views > 1 else 0)
+        if form not in seen:
+            seen.add(form)
+            out.append(c)
+    return out
+
+
 def measure(sa, device, base, scene_loader, poses, width: int, height: int, cand: Candidate,
             steps: int = 3, in_flight: int = 1, reps: int = 2) -> float:
     """frames/s of `steps` graph-replayed batches of cand.max_views views
@@ -82,13 +105,7 @@ def measure(sa, device, base, scene_loader, poses, width: int, height: int, cand
     frames.  One renderer runs on the device stream.  With more than one,
     each runs on a stream of its own: batches on the device stream did not
     overlap with those of an own-stream renderer, measured on MI355X."""
-    cfg = type(base)(**{k: getattr(base, k) for k in base.__dataclass_fields__})
-    cfg.radix_bits_per_digit = cand.radix_bits_per_digit
-    cfg.sort_tile_keys = cand.sort_tile_keys
-    cfg.max_views = cand.max_views
-    cfg.raster_mode = cand.raster_mode
-    cfg.raster_batch = cand.raster_batch
-    cfg.raster_longest_first = cand.raster_longest_first
+    cfg = configured(base, cand)
     rs = ([sa.Renderer(device, cfg)] if in_flight <= 1 else
           [sa.Renderer(device, cfg, own_stream=True) for _ in range(in_flight)])
     try:
@@ -124,10 +141,13 @@ def measure(sa, device, base, scene_loader, poses, width: int, height: int, cand
 
 
 def autotune(sa, device, base, scene_loader, poses, width: int, height: int, cands=None, steps: int = 3,
-             log=None) -> TuneResult:
+             log=None, splats: int | None = None) -> TuneResult:
     """Times every candidate; scene_loader(renderer) returns the scene to
-    render (it may return the same resident scene every time)."""
+    render (it may return the same resident scene every time).  splats: the
+    scene's size, where known, leaves repeats out (distinct)."""
     cands = cands or candidates()
+    if splats is not None:
+        cands = distinct(sa, base, cands, splats)
     table = []
     for c in cands:
         fps = measure(sa, device, base, scene_loader, poses, width, height, c, steps)
@@ -170,18 +190,22 @@ TIE = 0.03
 
 
 def autotune_staged(sa, device, base, scene_loader, poses, width: int, height: int, views: int, steps: int = 3,
-                    log=None, walk=(3, 0), in_flight: int = 1, tie: float = TIE) -> TuneResult:
+                    log=None, walk=(3, 0), in_flight: int = 1, tie: float = TIE,
+                    splats: int | None = None) -> TuneResult:
     """Coordinate search: the sort's digit width x tile with the raster at
-    its defaults, then the raster's batch x tile order (x walk) with the best
+    its defaults, then the raster's batch (x walk) with the best
     sort, at a fixed batch width and number of batches in flight.  Each stage
     tries its candidates in order of preference (larger sort tiles, which
     pay their look-back over more keys, and the raster's default form
     first); a later one is picked only if it beats the pick by more than
-    `tie`."""
+    `tie`.  splats: the scene's size, where known, leaves repeats out
+    (distinct)."""
     table = []
 
     def run(cands):
         pick = None
+        if splats is not None:
+            cands = distinct(sa, base, cands, splats)
         for c in cands:
             fps = measure(sa, device, base, scene_loader, poses, width, height, c, steps, in_flight)
             table.append((c.key(), round(fps, 2)))
@@ -194,6 +218,5 @@ def autotune_staged(sa, device, base, scene_loader, poses, width: int, height: i
     start = Candidate(8, 4096, views, walk[0], base.raster_batch, 0)
     c, _ = run([start.replace(radix_bits_per_digit=r, sort_tile_keys=t)
                 for t in sorted(SORT_TILE_KEYS, reverse=True) for r in sorted(RADIX_BITS, reverse=True)])
-    c, fps = run([c.replace(raster_batch=b, raster_longest_first=o, raster_mode=w)
-                  for b in RASTER_BATCH for o in RASTER_LONGEST_FIRST for w in walk])
+    c, fps = run([c.replace(raster_batch=b, raster_mode=w) for b in RASTER_BATCH for w in walk])
     return TuneResult(c, round(fps, 2), table)

@@ -265,25 +265,14 @@ int ensure_tile_work(spl_renderer* r, uint32_t tiles) {
   return SPL_OK;
 }
 
-// The whole pipeline for one batch, as a sequence of launches on `q`.
-// Every stage clears the bookkeeping of an earlier stage once that stage is
-// done (status words, histograms, tile ranges), so the sequence needs no
-// memset and replays as a graph.
-void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEvent_t* ev) {
-  const spl_configuration& cfg = r->cfg;
-  const spl_scene* s = b.scene;
-  const uint32_t n = (uint32_t)b.n, nv = b.views;
-  const bool sorted = cfg.depth_sorting != SPL_DEPTH_SORTING_NONE;
-  const int P = sorted ? r->depth_passes : 0;
-  const int bits = r->depth_bits;
-  const int radix = 1 << bits;
-  const int Q = b.pair_passes;
-  int tile_bits = 1;  // bits of the largest tile key, max_tiles - 1
-  while (tile_bits < 31 && (b.max_tiles - 1u) >> tile_bits) ++tile_bits;
-  const uint32_t cus = (uint32_t)r->dev->cu_count;
-  const uint32_t per_view = std::max<uint32_t>(1, cus * 4 / nv);
-  // radix-sort tiles: one 1024-lane, two 512-lane or four 256-lane blocks per CU, shared
-  // by the views (which sort side by side, so their look-back chains overlap)
+// Keys per radix-sort tile of a batch's depth and pair sorts, and whether
+// their keys are so few that lanes take fewer of them each.
+struct SortForm {
+  int depth_tile, pair_tile;
+  bool few;
+};
+
+SortForm sort_form(const spl_renderer* r, uint32_t n, uint32_t nv) {
   // A single view picks its tile by the scene's size, whatever the batches
   // use (the autotuner picks the batches' tile).  Small scenes leave CUs idle
   // and pay for a tile's own chain, large ones for the look-back over many
@@ -304,10 +293,35 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   // 32M splats, depth sort 5.19, 4.66 and 4.36 ms in 4096-, 8192- and
   // 16384-key tiles, pair sort 12.4, 11.8 and 12.4.
   const bool large = n > 1u << 22;
-  const int depth_tile = nv == 1 ? one_view(kSmallSort, 1u << 21, 1u << 22) : large ? 16384 : r->sort_tile;
-  const int pair_tile = nv == 1 ? one_view(small_pairs ? kSmallPairs : 0, 1u << 19, 1u << 21)
-                                : std::max(r->sort_tile, large ? 8192 : 0);
-  const int few_keys = nv == 1 || (uint64_t)n * nv <= 1u << 21;
+  SortForm f;
+  f.depth_tile = nv == 1 ? one_view(kSmallSort, 1u << 21, 1u << 22) : large ? 16384 : r->sort_tile;
+  f.pair_tile = nv == 1 ? one_view(small_pairs ? kSmallPairs : 0, 1u << 19, 1u << 21)
+                        : std::max(r->sort_tile, large ? 8192 : 0);
+  f.few = nv == 1 || (uint64_t)n * nv <= 1u << 21;
+  return f;
+}
+
+// The whole pipeline for one batch, as a sequence of launches on `q`.
+// Every stage clears the bookkeeping of an earlier stage once that stage is
+// done (status words, histograms, tile ranges), so the sequence needs no
+// memset and replays as a graph.
+void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEvent_t* ev) {
+  const spl_configuration& cfg = r->cfg;
+  const spl_scene* s = b.scene;
+  const uint32_t n = (uint32_t)b.n, nv = b.views;
+  const bool sorted = cfg.depth_sorting != SPL_DEPTH_SORTING_NONE;
+  const int P = sorted ? r->depth_passes : 0;
+  const int bits = r->depth_bits;
+  const int radix = 1 << bits;
+  const int Q = b.pair_passes;
+  int tile_bits = 1;  // bits of the largest tile key, max_tiles - 1
+  while (tile_bits < 31 && (b.max_tiles - 1u) >> tile_bits) ++tile_bits;
+  const uint32_t cus = (uint32_t)r->dev->cu_count;
+  const uint32_t per_view = std::max<uint32_t>(1, cus * 4 / nv);
+  const SortForm form = sort_form(r, n, nv);
+  // blocks of a sort pass: by its tile, one of 16384 keys, two of 8192 or
+  // four of less per CU, shared by the views (which sort side by side, so
+  // their look-back chains overlap)
   const auto sort_grid = [&](uint64_t keys, int tile) {
     const uint32_t per_view = std::max<uint32_t>(1, cus * 4 / std::max(1, tile / kSortTile) / nv);
     return (int)std::max<uint64_t>(1, std::min<uint64_t>(div_up(keys, (uint64_t)tile), per_view));
@@ -315,7 +329,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   const size_t cap = r->cap;
   const size_t sort_stride = r->sort_words * kMaxDepthPasses;
   const size_t pair_stride_status = r->pair_words * kMaxPairPasses;
-  const size_t sort_used = (size_t)div_up(n, depth_tile) * radix;
+  const size_t sort_used = (size_t)div_up(n, form.depth_tile) * radix;
   const size_t cull_used = div_up(n, kCullTile);
   auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], q); };
   // A sorted batch projects on the side stream while the depth sort runs
@@ -424,9 +438,9 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_words = cull_used;
       a.clear_a_stride = r->cull_tiles;
     }
-    a.tile_keys = depth_tile;
-    a.few = few_keys;
-    a.grid_x = sort_grid(n, depth_tile);
+    a.tile_keys = form.depth_tile;
+    a.few = form.few;
+    a.grid_x = sort_grid(n, form.depth_tile);
     a.views = (int)nv;
     // keys are below 2^30 (0 < clip.z < 1): the last 8-bit pass needs 6 bits
     launch_sort_pass(std::min(bits, 30 - p * bits), a, q);
@@ -488,12 +502,12 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     } else {
       a.clear_a = r->pair_status + (size_t)(p - 1) * r->pair_words;
       a.clear_a_words = r->pair_words;
-      a.clear_a_tile = (uint32_t)pair_tile;
+      a.clear_a_tile = (uint32_t)form.pair_tile;
       a.clear_a_stride = pair_stride_status;
     }
-    a.tile_keys = pair_tile;
-    a.few = few_keys;
-    a.grid_x = sort_grid(r->pair_cap, pair_tile);
+    a.tile_keys = form.pair_tile;
+    a.few = form.few;
+    a.grid_x = sort_grid(r->pair_cap, form.pair_tile);
     a.views = (int)nv;
     // tile keys are below max_tiles: the last pass takes only their top bits
     launch_sort_pass(std::max(5, std::min(8, tile_bits - 8 * p)), a, q);
@@ -509,7 +523,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.ranges = r->ranges; a.ranges_stride = r->ranges_cap;
     a.clear_a = r->pair_status + (size_t)(Q - 1) * r->pair_words;
     a.clear_a_words = r->pair_words;
-    a.clear_a_tile = (uint32_t)pair_tile;
+    a.clear_a_tile = (uint32_t)form.pair_tile;
     a.clear_a_stride = pair_stride_status;
     a.clear_b = r->pair_hist;
     a.clear_b_words = kHistCopies * kPairHist;
@@ -976,6 +990,23 @@ int spl_render_frame(spl_renderer* r, spl_scene* s, spl_frame* f, const float ca
 // ---------------------------------------------------------------------------
 // Parity and timing taps
 // ---------------------------------------------------------------------------
+
+int spl_debug_sort_tiles(const spl_configuration* cfg, uint64_t splats, uint32_t views, uint32_t* depth_tile_keys,
+                         uint32_t* pair_tile_keys) {
+  if (!cfg || !depth_tile_keys || !pair_tile_keys)
+    return fail(SPL_ERROR_INVALID_ARGUMENT, "spl_debug_sort_tiles: null argument");
+  const int rc = validate_config(cfg);
+  if (rc) return rc;
+  if (splats > cfg->max_splat_count) return fail(SPL_ERROR_CAPACITY, "scene has more splats than max_splat_count");
+  if (views == 0 || views > std::max<uint32_t>(1, cfg->max_views))
+    return fail(SPL_ERROR_INVALID_ARGUMENT, "spl_debug_sort_tiles: views must be in 1..=max_views");
+  spl_renderer r;  // sizes only: nothing is allocated
+  size_workspace(&r, cfg, cfg->max_splat_count, 0);
+  const SortForm f = sort_form(&r, (uint32_t)splats, views);
+  *depth_tile_keys = (uint32_t)f.depth_tile;
+  *pair_tile_keys = (uint32_t)f.pair_tile;
+  return SPL_OK;
+}
 
 int spl_debug_select_view(spl_renderer* r, uint32_t view) {
   if (!r) return fail(SPL_ERROR_INVALID_ARGUMENT, "null argument");
