@@ -65,12 +65,18 @@ def test_server_mix_equals_alone_and_plain():
     scenes, records = make_scenes(server)
     reqs = requests(16, seed=5)
     # A first pass of the same requests creates the slots, frames and launch
-    # graphs, so the measured burst below is submitted faster than the device
-    # renders it: requests then wait for a slot and leave in batches.
+    # graphs.
     for t in [server.submit(scenes[s], w, h, cam, view) for s, w, h, (cam, view) in reqs]:
         server.wait(t)
         server.release(t)
     warm = server.stats()
+    # Batches start behind the device stream's work: with some milliseconds of
+    # it queued, the burst below is submitted before any batch is done, however
+    # fast the device or slow the host, and what finds no slot leaves in batches.
+    r = sa.Renderer(device(), config(max_splat_count=1 << 17))
+    f = sa.Frame(device(), 640, 480)
+    for _ in range(64):
+        r.render_frame(f, *reqs[0][3], scenes[2])
     tickets = [server.submit(scenes[s], w, h, cam, view) for s, w, h, (cam, view) in reqs]
     mixed = []
     for t in tickets:
