@@ -272,31 +272,45 @@ struct SortForm {
   bool few;
 };
 
+// A single view picks its tiles by the scene's size, whatever the batches use
+// (the autotuner picks the batches' tile).  Few keys leave CUs idle and pay
+// for a tile's own chain, many for the look-back over many tiles; us, one view
+// on MI355X, depth sort in tiles of 1024, 4096, 8192 and 16384 keys (of 256 x
+// 4, 512 x 8, 1024 x 8 and 1024 x 16 lanes x keys):
+//             8-bit digits                10-bit digits
+//   1k     25    30    36    52        28    29    33    46
+//   20k    33    39    46    63        49    39    44    56
+//   65k    40    43    48    68        66    45    47    62
+//   100k   41    42    48    69        76    46    48    63
+//   131k   46    43    51    68        84    49    49    63
+//   700k         57    58    75              72    59    70
+//   1.2M         67    67    82              85    67    76
+//   2M           86    78    90             113    77    83
+//   3M          114   112    97             152   111    90
+//   6M          167   140   145             238   149   136
+// A 1024-key tile of 10-bit digits clears, publishes and looks back over as
+// many digits as it has keys.  Up to 2^21 keys 8192-key tiles go in one round
+// of blocks, beyond they take a second.
 SortForm sort_form(const spl_renderer* r, uint32_t n, uint32_t nv) {
-  // A single view picks its tile by the scene's size, whatever the batches
-  // use (the autotuner picks the batches' tile).  Small scenes leave CUs idle
-  // and pay for a tile's own chain, large ones for the look-back over many
-  // tiles; us, one view on MI355X, depth sort / pair sort in tiles of 1024,
-  // 4096, 8192 and 16384 keys:
-  //   20k splats   31 / 11    54 / 16     58 / 17    72 / 22
-  //   100k         40 / 34    51 / 31     59 / 32    75 / 38
-  //   1M           77 / 72    55 / 39     58 / 36    79 / 43
-  //   1.5M         96 / 74    61 / 41     60 / 37    79 / 44
-  //   3M at 4K    158 / 187   83 / 90     77 / 82    91 / 79
-  //   6M          232 / 217  116 / 100   107 / 90    98 / 85
-  // (20k and 100k in 4096- and 8192-key tiles: of 256 x 16 and 512 x 16 lanes)
-  const auto one_view = [n](uint64_t small, uint64_t narrow, uint64_t wide) {
-    return n <= small ? kSortTileSmall : n <= narrow ? kSortTile : n <= wide ? 8192 : 16384;
-  };
+  // The pair sort, in the same tiles: 20k splats 11, 16, 17 and 22 us, 100k
+  // 34, 31, 32 and 38, 1M 72, 39, 36 and 43, 1.5M 74, 41, 37 and 44, 3M at 4K
+  // 187, 90, 82 and 79, 6M 217, 100, 90 and 85.
   const bool small_pairs = r->pair_words >= (size_t)div_up(r->pair_cap, kSortTileSmall) * 256;
   // Batches of large scenes sort in larger tiles than configured: 8 views of
   // 32M splats, depth sort 5.19, 4.66 and 4.36 ms in 4096-, 8192- and
   // 16384-key tiles, pair sort 12.4, 11.8 and 12.4.
   const bool large = n > 1u << 22;
   SortForm f;
-  f.depth_tile = nv == 1 ? one_view(kSmallSort, 1u << 21, 1u << 22) : large ? 16384 : r->sort_tile;
-  f.pair_tile = nv == 1 ? one_view(small_pairs ? kSmallPairs : 0, 1u << 19, 1u << 21)
-                        : std::max(r->sort_tile, large ? 8192 : 0);
+  if (nv > 1) {
+    f.depth_tile = large ? 16384 : r->sort_tile;
+    f.pair_tile = std::max(r->sort_tile, large ? 8192 : 0);
+  } else {
+    const bool small = r->depth_bits == 8 && n <= kSmallSort;
+    f.depth_tile = small ? kSortTileSmall
+                   : n <= (r->depth_bits == 8 ? 1u << 20 : 1u << 17) ? kSortTile : n <= 1u << 21 ? 8192 : 16384;
+    f.pair_tile = small_pairs && n <= kSmallPairs ? kSortTileSmall
+                  : n <= 1u << 19 ? kSortTile : n <= 1u << 21 ? 8192 : 16384;
+  }
   f.few = nv == 1 || (uint64_t)n * nv <= 1u << 21;
   return f;
 }
@@ -747,7 +761,7 @@ void size_workspace(spl_renderer* r, const spl_configuration* cfg, uint64_t cap,
     return (size_t)std::max<uint64_t>(div_up(keys, kSortTile),
                                       std::min<uint64_t>(div_up(keys, kSortTileSmall), small / kSortTileSmall));
   };
-  r->sort_words = sort_tiles(r->cap, kSmallSort) * radix;
+  r->sort_words = sort_tiles(r->cap, r->depth_bits == 8 ? kSmallSort : 0) * radix;
   r->bin_words = div_up(r->cap, kBinThreads);
   r->pair_words = sort_tiles(r->pair_cap, 1u << 20) * 256;
 }

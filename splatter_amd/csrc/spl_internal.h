@@ -94,7 +94,8 @@ constexpr float kShConstants[16] = {
 constexpr int kCullThreads = 256, kCullItems = 16;   // 4096 splats per cull / project tile
 constexpr int kSortTile = 4096;                      // keys per sort tile: 4096, 8192 or 16384,
 constexpr int kSortTileSmall = 1024;                 // or these, for one view of a small scene:
-constexpr uint32_t kSmallSort = 1u << 17, kSmallPairs = 1u << 15;  // its splats (depth sort, pair sort)
+constexpr uint32_t kSmallSort = 7u << 14;            // its splats (depth sort, 8-bit digits)
+constexpr uint32_t kSmallPairs = 1u << 15;           // and (pair sort)
 constexpr int kBinThreads = 256, kBinItems = 4;      // 1024 draw ranks per bin tile, 256 in small batches
 constexpr uint32_t kHistCopies = 8;                  // of each view's digit histograms, summed by the sort
 constexpr int kCullTile = kCullThreads * kCullItems;

@@ -62,10 +62,12 @@ def test_blocks_that_share_a_cull_tile(count, views):
         assert normwise_rel(rec[:, 4:], orec[:, 4:]).max() <= RECORD_TOL
 
 
-# one view sorts depths in 1024-key tiles up to 2^17 splats, in 4096-key tiles
-# up to 2^19, in 8192-key tiles up to 2^22 and in 16384-key tiles beyond; pairs
-# change at 2^15, 2^18 and 2^21
-@pytest.mark.parametrize("count", [1000, 1 << 15, (1 << 15) + 1, 1 << 17, (1 << 17) + 1, 1 << 18, (1 << 18) + 1, 1 << 19, (1 << 19) + 1, (1 << 21) + 1, (1 << 22) + 1])
+# the sizes at which one view's depth sort (test_sort_tiles.py has its lines) and
+# pair sort (2^15, 2^19, 2^21 splats) change their tiles, and where a batch's do
+# (2^22)
+@pytest.mark.parametrize("count", [1000, 1 << 15, (1 << 15) + 1, 7 << 14, (7 << 14) + 1, 1 << 17, (1 << 17) + 1,
+                                   1 << 19, (1 << 19) + 1, 1 << 20, (1 << 20) + 1, 1 << 21, (1 << 21) + 1,
+                                   (1 << 22) + 1])
 @pytest.mark.parametrize("bits", [8, 10])
 def test_sort_tile_of_one_view(count, bits):
     say(f"{count} splats, {bits}-bit digits")
@@ -83,7 +85,7 @@ def test_sort_tile_of_one_view(count, bits):
     keys, idx = r.read_entries()
     okeys, oidx = ob.cpu_depth_sort(centers, ob.vp_of(ob.uniforms(cam, view, 640, 360)), 1.1)
     assert np.array_equal(idx, oidx) and np.array_equal(keys, okeys)
-    # a batch sorts its pairs in the configured tile: the same lists, the same image
+    # a batch of the view twice, in the batches' tiles: the same lists, the same image
     r.render_views(frames[::-1], [cam] * 2, [view] * 2, scene)
     assert np.array_equal(frames[0].read(), frames[1].read())
     batch = frames[0].read()
