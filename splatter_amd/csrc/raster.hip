@@ -346,7 +346,7 @@ __global__ __launch_bounds__(256) void k_tile_ranges(RangesLaunch a) {
   const uint32_t v = blockIdx.y;
   if (a.clear_a)
     clear_words(a.clear_a + v * a.clear_a_stride,
-                used_status(a.clear_a_words, a.clear_a_tile, a.counters[(size_t)v * kCounterWords + kPairs]));
+                used_status(a.clear_a_words, a.clear_a_tile, a.one_round, a.counters[(size_t)v * kCounterWords + kPairs]));
   if (a.clear_b) clear_words(a.clear_b + v * a.clear_b_stride, a.clear_b_words);
   if (blockIdx.x == 0 && v == 0 && threadIdx.x <= kHeavyClasses + 1) a.counters[kHeavyAll + threadIdx.x] = 0u;
   const uint32_t* keys = a.pair_keys + v * a.pair_stride;  // 16-byte aligned: pair_stride % 4 == 0

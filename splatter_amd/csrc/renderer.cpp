@@ -269,11 +269,11 @@ int ensure_tile_work(spl_renderer* r, uint32_t tiles) {
 // their keys are so few that lanes take fewer of them each.
 struct SortForm {
   int depth_tile, pair_tile;
-  bool few;
+  bool few, few_pairs;
 };
 
-// A single view picks its tiles by the scene's size, whatever the batches use
-// (the autotuner picks the batches' tile).  Few keys leave CUs idle and pay
+// A single view picks its tiles by its keys, whatever the batches use (the
+// autotuner picks the batches' tile).  Few keys leave CUs idle and pay
 // for a tile's own chain, many for the look-back over many tiles; us, one view
 // on MI355X, depth sort in tiles of 1024, 4096, 8192 and 16384 keys (of 256 x
 // 4, 512 x 8, 1024 x 8 and 1024 x 16 lanes x keys):
@@ -291,27 +291,51 @@ struct SortForm {
 // A 1024-key tile of 10-bit digits clears, publishes and looks back over as
 // many digits as it has keys.  Up to 2^21 keys 8192-key tiles go in one round
 // of blocks, beyond they take a second.
+//
+// How many pairs those are is not known before the frame: a splat of the same
+// scene has two at 1080p, forty at 4K.  Of 2^19 to 2^21 splats, and of fewer
+// whose renderer has room for more than 2^22 pairs, the pass reads the number
+// and takes 8192-key tiles while one round of blocks holds them, else 16384
+// (by_count_tile); us in tiles of 1024, 4096, 8192, 16384 and by count:
+//   61k pairs          21    23    25    36
+//   100k               23    23    25    36
+//   306k               33    26    27    37
+//   592k                     31    30    39    30
+//   1.4M                     42    38    44    39
+//   2.0M                     49    41    47    43
+//   2.4M                     62    60    49    50
+//   4.0M                     73    66    53    53
+//   9.8M                    139   117   113   114
+//   27M                     342   302   254   253
+// (beyond 2^21 splats 16384 without asking: 6M splats, 11.8M pairs, 117 us
+// against 120 by count.)
 SortForm sort_form(const spl_renderer* r, uint32_t n, uint32_t nv) {
-  // The pair sort, in the same tiles: 20k splats 11, 16, 17 and 22 us, 100k
-  // 34, 31, 32 and 38, 1M 72, 39, 36 and 43, 1.5M 74, 41, 37 and 44, 3M at 4K
-  // 187, 90, 82 and 79, 6M 217, 100, 90 and 85.
-  const bool small_pairs = r->pair_words >= (size_t)div_up(r->pair_cap, kSortTileSmall) * 256;
   // Batches of large scenes sort in larger tiles than configured: 8 views of
   // 32M splats, depth sort 5.19, 4.66 and 4.36 ms in 4096-, 8192- and
   // 16384-key tiles, pair sort 12.4, 11.8 and 12.4.
   const bool large = n > 1u << 22;
+  const uint64_t room = r->pair_cap * n / r->cap;  // the splats' share of the pair capacity
   SortForm f;
   if (nv > 1) {
-    f.depth_tile = large ? 16384 : r->sort_tile;
-    f.pair_tile = std::max(r->sort_tile, large ? 8192 : 0);
+    f.depth_tile = large ? kTileWide : r->sort_tile;
+    f.pair_tile = std::max(r->sort_tile, large ? kTileNarrow : 0);
   } else {
     const bool small = r->depth_bits == 8 && n <= kSmallSort;
-    f.depth_tile = small ? kSortTileSmall
-                   : n <= (r->depth_bits == 8 ? 1u << 20 : 1u << 17) ? kSortTile : n <= 1u << 21 ? 8192 : 16384;
-    f.pair_tile = small_pairs && n <= kSmallPairs ? kSortTileSmall
-                  : n <= 1u << 19 ? kSortTile : n <= 1u << 21 ? 8192 : 16384;
+    f.depth_tile = small                                             ? kSortTileSmall
+                   : n <= (r->depth_bits == 8 ? 1u << 20 : 1u << 17) ? kSortTile
+                   : n <= 1u << 21                                   ? kTileNarrow
+                                                                     : kTileWide;
+    const bool small_words = r->pair_words >= (size_t)div_up(r->pair_cap, kSortTileSmall) * 256;
+    f.pair_tile = small_words && n <= kSmallPairs && room <= 1u << 18 ? kSortTileSmall
+                  : n <= 1u << 19 && room <= 1u << 22                 ? kSortTile
+                  : n <= 1u << 21                                     ? kTileByCount
+                                                                      : kTileWide;
   }
+  // (batches: sort.hip has the figures of few keys.  Room for more than eight
+  // pairs a splat is taken for many pairs: sixteen views of 100k large splats,
+  // 1.4M pairs each, 14.9 us a view with eight keys a lane, 13.3 with sixteen.)
   f.few = nv == 1 || (uint64_t)n * nv <= 1u << 21;
+  f.few_pairs = f.few && (nv == 1 || room * nv <= 1u << 24);
   return f;
 }
 
@@ -333,16 +357,18 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   const uint32_t cus = (uint32_t)r->dev->cu_count;
   const uint32_t per_view = std::max<uint32_t>(1, cus * 4 / nv);
   const SortForm form = sort_form(r, n, nv);
-  // blocks of a sort pass: by its tile, one of 16384 keys, two of 8192 or
-  // four of less per CU, shared by the views (which sort side by side, so
-  // their look-back chains overlap)
+  // blocks of a sort pass: by its tile, one of 16384 keys (or by count), two
+  // of 8192 or four of less per CU, shared by the views (which sort side by
+  // side, so their look-back chains overlap)
   const auto sort_grid = [&](uint64_t keys, int tile) {
-    const uint32_t per_view = std::max<uint32_t>(1, cus * 4 / std::max(1, tile / kSortTile) / nv);
-    return (int)std::max<uint64_t>(1, std::min<uint64_t>(div_up(keys, (uint64_t)tile), per_view));
+    const int least = tile == kTileByCount ? kTileNarrow : tile, most = tile == kTileByCount ? kTileWide : tile;
+    const uint32_t per_view = std::max<uint32_t>(1, cus * 4 / std::max(1, most / kSortTile) / nv);
+    return (int)std::max<uint64_t>(1, std::min<uint64_t>(div_up(keys, (uint64_t)least), per_view));
   };
   const size_t cap = r->cap;
   const size_t sort_stride = r->sort_words * kMaxDepthPasses;
   const size_t pair_stride_status = r->pair_words * kMaxPairPasses;
+  const uint32_t one_round = cus * (uint32_t)kTileNarrow;
   const size_t sort_used = (size_t)div_up(n, form.depth_tile) * radix;
   const size_t cull_used = div_up(n, kCullTile);
   auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], q); };
@@ -520,7 +546,8 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_stride = pair_stride_status;
     }
     a.tile_keys = form.pair_tile;
-    a.few = form.few;
+    a.one_round = one_round;
+    a.few = form.few_pairs;
     a.grid_x = sort_grid(r->pair_cap, form.pair_tile);
     a.views = (int)nv;
     // tile keys are below max_tiles: the last pass takes only their top bits
@@ -538,6 +565,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
     a.clear_a = r->pair_status + (size_t)(Q - 1) * r->pair_words;
     a.clear_a_words = r->pair_words;
     a.clear_a_tile = (uint32_t)form.pair_tile;
+    a.one_round = one_round;
     a.clear_a_stride = pair_stride_status;
     a.clear_b = r->pair_hist;
     a.clear_b_words = kHistCopies * kPairHist;
@@ -1018,7 +1046,7 @@ int spl_debug_sort_tiles(const spl_configuration* cfg, uint64_t splats, uint32_t
   size_workspace(&r, cfg, cfg->max_splat_count, 0);
   const SortForm f = sort_form(&r, (uint32_t)splats, views);
   *depth_tile_keys = (uint32_t)f.depth_tile;
-  *pair_tile_keys = (uint32_t)f.pair_tile;
+  *pair_tile_keys = f.pair_tile == kTileByCount ? 0u : (uint32_t)f.pair_tile;
   return SPL_OK;
 }
 

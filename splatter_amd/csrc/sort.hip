@@ -8,7 +8,7 @@
 //    bumped by the lowest peer) carries the rank across the wave's items.
 //    Items are visited in input order, so the pass is stable -- the
 //    reference ranks with LDS atomicAdd (shaders.wgsl:428-429), which is not.
-//  - tiles are TILE = THREADS*ITEMS keys (1024 to 16384) taken in order from an
+//  - tiles are THREADS*ITEMS keys (1024 to 16384) taken in order from an
 //    atomic counter by a persistent grid (reference: 1024-key tiles, one
 //    workgroup each, shaders.wgsl:406-420); full tiles skip every per-key
 //    bounds test.
@@ -32,14 +32,21 @@ struct Flag {
   static constexpr bool value = B;
 };
 
-template <int BITS, int THREADS, int ITEMS>
+template <int N>
+struct Int {
+  static constexpr int value = N;
+};
+
+// NARROW > 0: the pass takes NARROW keys a lane instead of ITEMS where its
+// keys are at most a.one_round, read on the device (by_count_tile).
+template <int BITS, int THREADS, int ITEMS, int NARROW = 0>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_onesweep_pass(SortPassLaunch a) {
   constexpr int RADIX = 1 << BITS;
   constexpr int WAVES = THREADS / kWave;
-  constexpr int TILE = THREADS * ITEMS;
+  static_assert(NARROW == 0 || (THREADS * NARROW == kTileNarrow && THREADS * ITEMS == kTileWide), "by_count_tile");
   constexpr int DPT = (RADIX + THREADS - 1) / THREADS;  // digits per thread
   constexpr uint32_t MASK = RADIX - 1;
-  __shared__ uint32_t s_buf[TILE];
+  __shared__ uint32_t s_buf[THREADS * ITEMS];
   __shared__ uint32_t s_wave_hist[WAVES * RADIX];
   __shared__ uint32_t s_digit_start[RADIX];
   __shared__ uint32_t s_local[RADIX];
@@ -52,7 +59,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
   const uint32_t v = blockIdx.y;
   uint32_t* counters = a.counters + (size_t)v * kCounterWords;
   if (a.clear_a)
-    clear_words(a.clear_a + v * a.clear_a_stride, used_status(a.clear_a_words, a.clear_a_tile, counters[a.count_slot]));
+    clear_words(a.clear_a + v * a.clear_a_stride,
+                used_status(a.clear_a_words, a.clear_a_tile, a.one_round, counters[a.count_slot]));
   if (a.clear_b) clear_words(a.clear_b + v * a.clear_b_stride, a.clear_b_words);
   const uint32_t* keys_in = a.keys_in + v * a.entry_stride;
   const uint32_t* vals_in = a.vals_in ? a.vals_in + v * a.entry_stride : nullptr;
@@ -64,7 +72,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
 
   uint32_t n = counters[a.count_slot];
   if (n > a.count_cap) n = a.count_cap;
-  const uint32_t num_tiles = (n + TILE - 1) / TILE;
+  const uint32_t tile_keys = NARROW ? by_count_tile(n, a.one_round) : THREADS * ITEMS;
+  const uint32_t num_tiles = (n + tile_keys - 1) / tile_keys;
   if (persistent_idle(num_tiles)) return;
   const int shift = a.shift;
 
@@ -97,19 +106,20 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
 #pragma unroll
   for (int b = 0; b < BITS; ++b) bit_at[b] = (uint32_t)shift + (uint32_t)b;
 
-  // One tile.  FULL tiles (all but the last of a view) hold TILE keys and
-  // skip every per-key bounds test.
-  auto tile_pass = [&](auto full_tag, const uint32_t t, const uint32_t tile_n) {
+  // One tile of KEYS keys a lane.  FULL tiles (all but the last of a view)
+  // hold TILE keys and skip every per-key bounds test.
+  auto tile_pass = [&](auto full_tag, auto keys_tag, const uint32_t t, const uint32_t tile_n) {
     constexpr bool FULL = decltype(full_tag)::value;
+    constexpr int KEYS = decltype(keys_tag)::value, TILE = THREADS * KEYS;
     const uint32_t tile_base = t * TILE;
 
     // Register budget: keys die once they are in LDS, values are fetched
     // while the look-back waits, and the scatter keeps digits packed (four
     // 8-bit or two 16-bit to a register) instead of 32-bit positions.
-    uint32_t key[ITEMS], pos[ITEMS];
-    const uint32_t wave_base = tile_base + w * (kWave * ITEMS) + lane;
+    uint32_t key[KEYS], pos[KEYS];
+    const uint32_t wave_base = tile_base + w * (kWave * KEYS) + lane;
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
+    for (int j = 0; j < KEYS; ++j) {
       const uint32_t idx = wave_base + j * kWave;
       key[j] = FULL || idx < n ? keys_in[idx] : 0xFFFFFFFFu;
     }
@@ -121,7 +131,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     volatile __attribute__((address_space(3))) uint32_t* wh =
         (volatile __attribute__((address_space(3))) uint32_t*)(s_wave_hist + w * RADIX);
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
+    for (int j = 0; j < KEYS; ++j) {
       const bool valid = FULL || (wave_base + j * kWave) < n;
       const uint32_t d = (key[j] >> shift) & MASK;
       const uint64_t vm = FULL ? ~0ull : __ballot(valid);
@@ -188,16 +198,16 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
 
     // keys to their place in the tile, sorted by digit
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
+    for (int j = 0; j < KEYS; ++j) {
       if (FULL || wave_base + j * kWave < n) {
         const uint32_t d = (key[j] >> shift) & MASK;
         pos[j] += s_local[d] + s_wave_hist[w * RADIX + d];
         if (pos[j] < (uint32_t)TILE) s_buf[pos[j]] = key[j];
       }
     }
-    uint32_t val[ITEMS];
+    uint32_t val[KEYS];
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
+    for (int j = 0; j < KEYS; ++j) {
       const uint32_t idx = wave_base + j * kWave;
       val[j] = FULL || idx < n ? (vals_in ? vals_in[idx] : idx) : 0u;
     }
@@ -218,11 +228,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
 
     constexpr int PW = BITS <= 8 ? 8 : 16;  // bits per packed digit
     constexpr int PER = 32 / PW;
-    uint32_t dig[(ITEMS + PER - 1) / PER];
+    uint32_t dig[(KEYS + PER - 1) / PER];
 #pragma unroll
-    for (int k = 0; k < (ITEMS + PER - 1) / PER; ++k) dig[k] = 0u;
+    for (int k = 0; k < (KEYS + PER - 1) / PER; ++k) dig[k] = 0u;
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
+    for (int k = 0; k < KEYS; ++k) {
       const uint32_t i = k * THREADS + tid;
       if (FULL || i < tile_n) {
         const uint32_t kk = s_buf[i];
@@ -237,11 +247,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
+    for (int j = 0; j < KEYS; ++j)
       if ((FULL || wave_base + j * kWave < n) && pos[j] < (uint32_t)TILE) s_buf[pos[j]] = val[j];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
+    for (int k = 0; k < KEYS; ++k) {
       const uint32_t i = k * THREADS + tid;
       if (FULL || i < tile_n) {
         const uint32_t d = (dig[k / PER] >> (PW * (k % PER))) & ((1u << PW) - 1u);
@@ -252,17 +262,29 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     __syncthreads();
   };
 
-  while (true) {
-    if (tid == 0) s_tile = take_ticket(tile_counter, num_tiles);
-    for (int i = tid; i < WAVES * RADIX; i += THREADS) s_wave_hist[i] = 0u;
-    __syncthreads();
-    const uint32_t t = s_tile;
-    if (t >= num_tiles) break;
-    const uint32_t left = n - t * TILE;
-    if (left >= (uint32_t)TILE) tile_pass(Flag<true>{}, t, (uint32_t)TILE);
-    else tile_pass(Flag<false>{}, t, left);
-    if (one_tile_each(num_tiles)) break;
+  // (a loop of its own for each number of keys a lane: in one loop the
+  // compiler keeps what both need across tiles in registers)
+  const auto take_tiles = [&](auto keys_tag) {
+    constexpr uint32_t TILE = THREADS * decltype(keys_tag)::value;
+    while (true) {
+      if (tid == 0) s_tile = take_ticket(tile_counter, num_tiles);
+      for (int i = tid; i < WAVES * RADIX; i += THREADS) s_wave_hist[i] = 0u;
+      __syncthreads();
+      const uint32_t t = s_tile;
+      if (t >= num_tiles) break;
+      const uint32_t left = n - t * TILE;
+      if (left >= TILE) tile_pass(Flag<true>{}, keys_tag, t, TILE);
+      else tile_pass(Flag<false>{}, keys_tag, t, left);
+      if (one_tile_each(num_tiles)) break;
+    }
+  };
+  if constexpr (NARROW > 0) {
+    if (tile_keys != (uint32_t)(THREADS * ITEMS)) {
+      take_tiles(Int<NARROW>{});
+      return;
+    }
   }
+  take_tiles(Int<ITEMS>{});
 }
 
 // Lanes and keys a lane of each tile size.  Few keys in all (`few`): eight or
@@ -275,6 +297,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
 template <int BITS>
 void launch_sort_pass_as(const SortPassLaunch& a, hipStream_t s) {
   const dim3 grid(a.grid_x, a.views);
+  if constexpr (BITS <= 8) {  // (pairs only)
+    if (a.tile_keys == kTileByCount) {
+      hipLaunchKernelGGL((k_onesweep_pass<BITS, 1024, 16, 8>), grid, dim3(1024), 0, s, a);
+      return;
+    }
+  }
   if (a.tile_keys == 16384)
     hipLaunchKernelGGL((k_onesweep_pass<BITS, 1024, 16>), grid, dim3(1024), 0, s, a);
   else if (a.tile_keys == 8192 && a.few)

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "spl_internal.h"
+
 namespace spl {
 
 constexpr int kWave = 64;
@@ -191,10 +193,18 @@ __device__ __forceinline__ uint32_t take_ticket(uint32_t* counter, uint32_t num_
   return t;
 }
 
+// The tile of a pass over `count` keys that goes by their number: the smaller
+// while one round of blocks (one of 1024 lanes a CU, `one_round` keys) holds
+// them all.
+__device__ __forceinline__ uint32_t by_count_tile(uint32_t count, uint32_t one_round) {
+  return count <= one_round ? kTileNarrow : kTileWide;
+}
+
 // Words of a finished sort pass's status to zero: of the capacity's `words`,
 // those of the tiles (`tile` keys, at most 256 digits) that `count` keys had;
 // tile 0: all.
-__device__ __forceinline__ size_t used_status(size_t words, uint32_t tile, uint32_t count) {
+__device__ __forceinline__ size_t used_status(size_t words, uint32_t tile, uint32_t one_round, uint32_t count) {
+  if (tile == kTileByCount) tile = by_count_tile(count, one_round);
   const size_t used = tile ? ((size_t)count + tile - 1) / tile * 256 : words;
   return used < words ? used : words;
 }

@@ -96,6 +96,8 @@ constexpr int kSortTile = 4096;                      // keys per sort tile: 4096
 constexpr int kSortTileSmall = 1024;                 // or these, for one view of a small scene:
 constexpr uint32_t kSmallSort = 7u << 14;            // its splats (depth sort, 8-bit digits)
 constexpr uint32_t kSmallPairs = 1u << 15;           // and (pair sort)
+constexpr int kTileNarrow = 8192, kTileWide = 16384; // by_count_tile's two,
+constexpr int kTileByCount = 1;                      // asked for by this tile size
 constexpr int kBinThreads = 256, kBinItems = 4;      // 1024 draw ranks per bin tile, 256 in small batches
 constexpr uint32_t kHistCopies = 8;                  // of each view's digit histograms, summed by the sort
 constexpr int kCullTile = kCullThreads * kCullItems;
@@ -145,7 +147,8 @@ struct SortPassLaunch {
   uint32_t* clear_a; size_t clear_a_words; size_t clear_a_stride;
   uint32_t* clear_b; size_t clear_b_words; size_t clear_b_stride;
   uint32_t clear_a_tile;     // keys per tile of the status at clear_a (used_status); 0: clear_a_words it is
-  int tile_keys;             // 1024, 4096, 8192 or 16384
+  uint32_t one_round;        // keys of one round of 1024-lane blocks, one a CU, in tiles of kTileNarrow
+  int tile_keys;             // 1024, 4096, 8192, 16384 or kTileByCount
   int few;                   // few keys in all: more lanes with fewer keys each
   int grid_x, views;
 };
@@ -193,7 +196,7 @@ struct RangesLaunch {
   const Uniforms* uniforms;
   uint2* ranges; size_t ranges_stride;
   uint32_t* clear_a; size_t clear_a_words; size_t clear_a_stride;
-  uint32_t clear_a_tile;     // as in SortPassLaunch
+  uint32_t clear_a_tile, one_round;  // as in SortPassLaunch
   uint32_t* clear_b; size_t clear_b_words; size_t clear_b_stride;
   int grid_x, views;
 };

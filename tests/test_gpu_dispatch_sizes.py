@@ -7,7 +7,7 @@ import pytest
 import oracle_bind as ob
 import splatter_amd as sa
 from gpu_common import Case, config, device, image_diff, normwise_rel, say
-from splatter_amd.synth import Workload, sphere_pose
+from splatter_amd.synth import Workload, look_at, sphere_pose
 
 pytestmark = pytest.mark.gpu
 
@@ -91,6 +91,42 @@ def test_sort_tile_of_one_view(count, bits):
     batch = frames[0].read()
     r.render_frame(frames[0], cam, view, scene)
     assert np.array_equal(frames[0].read(), batch)
+
+
+# One view of 2^21 splats sorts its pairs in 8192-key tiles while one a CU holds
+# them (2^21 on 256 CUs) and in 16384-key ones beyond: one pair short, that many
+# and a few more, each splat but the first in the middle of a screen tile.
+@pytest.mark.parametrize("first", ["behind", "small", "large"])
+def test_pair_tile_by_count(first):
+    n, width, height = 1 << 21, 1280, 720
+    rng = np.random.default_rng(73)
+    z = rng.uniform(3.0, 6.0, n)
+    x = (2.0 * (16 * rng.integers(0, width // 16, n) + 8) / width - 1.0) * z * width / height
+    y = (2.0 * (16 * rng.integers(0, height // 16, n) + 8) / height - 1.0) * z
+    base = Workload("gaussian", 1 << 16, seed=73).all()
+    rec = np.tile(base, n // len(base))
+    rec["center"] = np.stack([x, y, z - 5.0], axis=1)
+    rec["scale"] = -4.5  # a pixel or two
+    if first == "behind":
+        rec["center"][0] = (0.0, 0.0, -20.0)
+    if first == "large":
+        rec["scale"][0] = -1.5
+    r = sa.Renderer(device(), config(max_splat_count=n, max_views=2, tile_pairs_per_splat=2))
+    assert sa.sort_tiles(r.config, n, 1)[1] == 0
+    scene = sa.Scene(r, n)
+    scene.load_records(0, rec)
+    cam, view = look_at((0, 0, -5), (0, 0, 0))
+    frames = [sa.Frame(device(), width, height) for _ in range(2)]
+    for _ in range(2):  # the second frame finds what the first one cleared
+        r.render_frame(frames[0], cam, view, scene)
+    img, pairs = frames[0].read(), r.pair_count()
+    say(f"first splat {first}: {pairs} pairs")
+    assert pairs == n - 1 if first == "behind" else pairs == n if first == "small" else n < pairs < n + 100
+    # a batch of the view twice sorts them in 4096-key tiles: the same image
+    r.render_views(frames[::-1], [cam] * 2, [view] * 2, scene)
+    assert r.pair_count() == pairs
+    assert np.array_equal(frames[0].read(), img) and np.array_equal(frames[1].read(), img)
+    assert img[..., :3].any()
 
 
 # A list of 512 pairs and 1/1000 of the frame's makes a tile heavy.  Lists from
