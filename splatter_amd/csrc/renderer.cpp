@@ -325,8 +325,7 @@ SortForm sort_form(const spl_renderer* r, uint32_t n, uint32_t nv) {
                    : n <= (r->depth_bits == 8 ? 1u << 20 : 1u << 17) ? kSortTile
                    : n <= 1u << 21                                   ? kTileNarrow
                                                                      : kTileWide;
-    const bool small_words = r->pair_words >= (size_t)div_up(r->pair_cap, kSortTileSmall) * 256;
-    f.pair_tile = small_words && n <= kSmallPairs && room <= 1u << 18 ? kSortTileSmall
+    f.pair_tile = r->pair_cap <= kSmallPairCap && n <= kSmallPairs && room <= 1u << 18 ? kSortTileSmall
                   : n <= 1u << 19 && room <= 1u << 22                 ? kSortTile
                   : n <= 1u << 21                                     ? kTileByCount
                                                                       : kTileWide;
@@ -784,14 +783,16 @@ void size_workspace(spl_renderer* r, const spl_configuration* cfg, uint64_t cap,
   r->pair_cap = std::min<uint64_t>(pair_cap, (1ull << 30) - (1ull << 20)) & ~3ull;
   if (r->pair_cap == 0) r->pair_cap = 4;
   r->cull_tiles = div_up(r->cap, kCullTile);
-  // tiles of 4096 keys, or as many of 1024 as a small scene has
+  // tiles of 4096 keys, or as many of 1024 as a pass may take (sort_form):
+  // depths of scenes up to kSmallSort, pairs where all that fit do
+  const uint64_t small_depths = r->depth_bits == 8 ? std::min<uint64_t>(r->cap, kSmallSort) : 0;
+  const uint64_t small_pairs = r->pair_cap <= kSmallPairCap ? r->pair_cap : 0;
   const auto sort_tiles = [](uint64_t keys, uint64_t small) {
-    return (size_t)std::max<uint64_t>(div_up(keys, kSortTile),
-                                      std::min<uint64_t>(div_up(keys, kSortTileSmall), small / kSortTileSmall));
+    return (size_t)std::max<uint64_t>(div_up(keys, kSortTile), div_up(small, kSortTileSmall));
   };
-  r->sort_words = sort_tiles(r->cap, r->depth_bits == 8 ? kSmallSort : 0) * radix;
+  r->sort_words = sort_tiles(r->cap, small_depths) * radix;
   r->bin_words = div_up(r->cap, kBinThreads);
-  r->pair_words = sort_tiles(r->pair_cap, 1u << 20) * 256;
+  r->pair_words = sort_tiles(r->pair_cap, small_pairs) * 256;
 }
 
 }  // namespace

@@ -95,7 +95,8 @@ constexpr int kCullThreads = 256, kCullItems = 16;   // 4096 splats per cull / p
 constexpr int kSortTile = 4096;                      // keys per sort tile: 4096, 8192 or 16384,
 constexpr int kSortTileSmall = 1024;                 // or these, for one view of a small scene:
 constexpr uint32_t kSmallSort = 7u << 14;            // its splats (depth sort, 8-bit digits)
-constexpr uint32_t kSmallPairs = 1u << 15;           // and (pair sort)
+constexpr uint32_t kSmallPairs = 1u << 15;           // and (pair sort, with a capacity
+constexpr uint32_t kSmallPairCap = 1u << 20;         // of no more pairs than this)
 constexpr int kTileNarrow = 8192, kTileWide = 16384; // by_count_tile's two,
 constexpr int kTileByCount = 1;                      // asked for by this tile size
 constexpr int kBinThreads = 256, kBinItems = 4;      // 1024 draw ranks per bin tile, 256 in small batches
