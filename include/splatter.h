@@ -300,9 +300,9 @@ int spl_debug_enable_timing(spl_renderer* renderer, int enable);
 int spl_debug_stage_times(spl_renderer* renderer, float* ms, uint32_t capacity);
 /* Keys per radix-sort tile that a renderer of `configuration` takes for the
  * depth sort and for the pair sort of a batch of `views` views of a scene of
- * `splats` splats, so that a report or a tuner can name what runs.  Pairs: 0
- * where the pass goes by their number, 8192-key tiles while one round of
- * blocks holds them (2^21 pairs on 256 CUs) and 16384-key ones beyond.  Needs
+ * `splats` splats, so that a report or a tuner can name what runs.  0: the
+ * sort goes by how many keys the frame has, 8192-key tiles while one round of
+ * blocks holds them (2^21 keys on 256 CUs) and 16384-key ones beyond.  Needs
  * no device. */
 int spl_debug_sort_tiles(const spl_configuration* configuration, uint64_t splats, uint32_t views,
                          uint32_t* depth_tile_keys, uint32_t* pair_tile_keys);

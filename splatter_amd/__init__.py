@@ -101,8 +101,8 @@ class Configuration:
 
 def sort_tiles(config: Configuration, splats: int, views: int) -> tuple[int, int]:
     """Keys per radix-sort tile of the depth sort and of the pair sort that a
-    batch of `views` views of a scene of `splats` splats runs with (pairs: 0
-    where the pass picks 8192 or 16384 by their number)."""
+    batch of `views` views of a scene of `splats` splats runs with (0: 8192 or
+    16384, by how many keys the frame has)."""
     depth, pairs = C.c_uint32(), C.c_uint32()
     c = config.to_c()
     check(lib().spl_debug_sort_tiles(C.byref(c), splats, views, C.byref(depth), C.byref(pairs)))

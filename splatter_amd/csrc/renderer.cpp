@@ -290,13 +290,16 @@ struct SortForm {
 //   6M          167   140   145             238   149   136
 // A 1024-key tile of 10-bit digits clears, publishes and looks back over as
 // many digits as it has keys.  Up to 2^21 keys 8192-key tiles go in one round
-// of blocks, beyond they take a second.
+// of blocks, beyond they take a second.  Of more than 2^21 splats the pass reads
+// how many are visible and takes 8192-key tiles while one round holds them,
+// else 16384 (by_count_tile): 1.6M of 3M visible 81 us, in 16384-key tiles 92.
+// (Not of fewer: that kernel has the 16384-key form's registers and LDS, which
+// leave the projection beside it less room; a frame of 700k 313 us, else 304.)
 //
 // How many pairs those are is not known before the frame: a splat of the same
 // scene has two at 1080p, forty at 4K.  Of 2^19 to 2^21 splats, and of fewer
-// whose renderer has room for more than 2^22 pairs, the pass reads the number
-// and takes 8192-key tiles while one round of blocks holds them, else 16384
-// (by_count_tile); us in tiles of 1024, 4096, 8192, 16384 and by count:
+// whose renderer has room for more than 2^22 pairs, the pass goes by their
+// number in the same way; us in tiles of 1024, 4096, 8192, 16384 and by count:
 //   61k pairs          21    23    25    36
 //   100k               23    23    25    36
 //   306k               33    26    27    37
@@ -307,8 +310,8 @@ struct SortForm {
 //   4.0M                     73    66    53    53
 //   9.8M                    139   117   113   114
 //   27M                     342   302   254   253
-// (beyond 2^21 splats 16384 without asking: 6M splats, 11.8M pairs, 117 us
-// against 120 by count.)
+// (beyond 2^21 splats 16384 without asking: 3M at 4K, 7.2M pairs, 86 us, by
+// count 88.)
 SortForm sort_form(const spl_renderer* r, uint32_t n, uint32_t nv) {
   // Batches of large scenes sort in larger tiles than configured: 8 views of
   // 32M splats, depth sort 5.19, 4.66 and 4.36 ms in 4096-, 8192- and
@@ -324,7 +327,7 @@ SortForm sort_form(const spl_renderer* r, uint32_t n, uint32_t nv) {
     f.depth_tile = small                                             ? kSortTileSmall
                    : n <= (r->depth_bits == 8 ? 1u << 20 : 1u << 17) ? kSortTile
                    : n <= 1u << 21                                   ? kTileNarrow
-                                                                     : kTileWide;
+                                                                     : kTileByCount;
     f.pair_tile = r->pair_cap <= kSmallPairCap && n <= kSmallPairs && room <= 1u << 18 ? kSortTileSmall
                   : n <= 1u << 19 && room <= 1u << 22                 ? kSortTile
                   : n <= 1u << 21                                     ? kTileByCount
@@ -368,7 +371,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
   const size_t sort_stride = r->sort_words * kMaxDepthPasses;
   const size_t pair_stride_status = r->pair_words * kMaxPairPasses;
   const uint32_t one_round = cus * (uint32_t)kTileNarrow;
-  const size_t sort_used = (size_t)div_up(n, form.depth_tile) * radix;
+  const size_t sort_used = (size_t)div_up(n, form.depth_tile == kTileByCount ? kTileNarrow : form.depth_tile) * radix;
   const size_t cull_used = div_up(n, kCullTile);
   auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], q); };
   // A sorted batch projects on the side stream while the depth sort runs
@@ -478,6 +481,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_stride = r->cull_tiles;
     }
     a.tile_keys = form.depth_tile;
+    a.one_round = one_round;
     a.few = form.few;
     a.grid_x = sort_grid(n, form.depth_tile);
     a.views = (int)nv;
@@ -1046,8 +1050,9 @@ int spl_debug_sort_tiles(const spl_configuration* cfg, uint64_t splats, uint32_t
   spl_renderer r;  // sizes only: nothing is allocated
   size_workspace(&r, cfg, cfg->max_splat_count, 0);
   const SortForm f = sort_form(&r, (uint32_t)splats, views);
-  *depth_tile_keys = (uint32_t)f.depth_tile;
-  *pair_tile_keys = f.pair_tile == kTileByCount ? 0u : (uint32_t)f.pair_tile;
+  const auto told = [](int tile) { return tile == kTileByCount ? 0u : (uint32_t)tile; };
+  *depth_tile_keys = told(f.depth_tile);
+  *pair_tile_keys = told(f.pair_tile);
   return SPL_OK;
 }
 

@@ -297,13 +297,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
 template <int BITS>
 void launch_sort_pass_as(const SortPassLaunch& a, hipStream_t s) {
   const dim3 grid(a.grid_x, a.views);
-  if constexpr (BITS <= 8) {  // (pairs only)
-    if (a.tile_keys == kTileByCount) {
-      hipLaunchKernelGGL((k_onesweep_pass<BITS, 1024, 16, 8>), grid, dim3(1024), 0, s, a);
-      return;
-    }
-  }
-  if (a.tile_keys == 16384)
+  if (a.tile_keys == kTileByCount)
+    hipLaunchKernelGGL((k_onesweep_pass<BITS, 1024, 16, 8>), grid, dim3(1024), 0, s, a);
+  else if (a.tile_keys == 16384)
     hipLaunchKernelGGL((k_onesweep_pass<BITS, 1024, 16>), grid, dim3(1024), 0, s, a);
   else if (a.tile_keys == 8192 && a.few)
     hipLaunchKernelGGL((k_onesweep_pass<BITS, 1024, 8>), grid, dim3(1024), 0, s, a);
