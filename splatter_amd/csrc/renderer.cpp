@@ -500,7 +500,7 @@ void launch_sequence(spl_renderer* r, const BatchShape& b, hipStream_t q, hipEve
       a.clear_a_words = sort_used;
       a.clear_a_stride = sort_stride;
       a.clear_b = r->depth_hist;
-      a.clear_b_words = kHistCopies * kDepthHist;
+      a.clear_b_words = cull_hist ? kHistCopies * kDepthHist : kDepthHist;  // a batch fills one copy a view
       a.clear_b_stride = kHistCopies * kDepthHist;
     }
     a.order = sorted ? r->vals[fin] : nullptr; a.order_stride = cap;
