@@ -86,10 +86,10 @@ def test_gaussian_1m_1080p_random_pose():
 @pytest.mark.parametrize("unaligned,blend", [(True, sa.BlendMode.UNORM8), (False, sa.BlendMode.UNORM8),
                                              (True, sa.BlendMode.F32), (False, sa.BlendMode.F32)])
 def test_single_view_split_heavy_tiles(unaligned, blend):
-    """One view in mode 3 gives each tile with a list of 8x the mean (and
-    2048 pairs) four blocks, one per quadrant: the frame still equals the
-    oracle's, and equals the same view rendered in a batch (no split)."""
-    say(f"split heavy tiles, unaligned {unaligned}, blend {blend}")
+    """Dense clusters put lists of 8x the mean and 2048 pairs, which have
+    blocks of their own, among the others: the frame equals the oracle's, and
+    equals the same view rendered in a batch, where the threshold is another."""
+    say(f"heavy tiles, unaligned {unaligned}, blend {blend}")
     case = Case(Workload("tight", 200_000, seed=12),
                 config(use_unaligned_rectangles=unaligned, blend_mode=blend, raster_mode=3, max_views=2),
                 800, 600, orbit_poses(8, radius=8)[5])
@@ -97,7 +97,7 @@ def test_single_view_split_heavy_tiles(unaligned, blend):
     img = check_case(case, conics=False)
     lens = case.renderer.tile_stats()[:, 0].astype(np.int64)
     heavy = np.count_nonzero(lens >= max(8 * (lens.sum() // len(lens)), 2048))
-    say(f"  tiles {len(lens)}, mean list {lens.mean():.0f}, max {lens.max()}, split tiles {heavy}")
+    say(f"  tiles {len(lens)}, mean list {lens.mean():.0f}, max {lens.max()}, heavy tiles {heavy}")
     assert heavy > 0
     other = sa.Frame(case.frame.device, case.width, case.height)
     case.renderer.render_views([case.frame, other], [case.cam, orbit_poses(8, radius=8)[1][0]],
@@ -140,12 +140,22 @@ def test_depth_sorting_none_draws_in_index_order():
     (10, 4096, 0, 256, 0), (8, 8192, 0, 128, 1), (10, 8192, 1, 128, 0), (8, 4096, 1, 256, 1),
     (8, 16384, 2, 128, 0), (10, 16384, 2, 256, 1), (10, 16384, 3, 128, 0), (8, 8192, 3, 256, 1)])
 def test_autotuner_options(bits, tile, mode, batch, longest):
-    # every option the autotuner may pick gives the same bit-exact order and image
+    # every option the autotuner may pick gives the same bit-exact order and
+    # image, in one view (which takes neither the sort tile nor the raster's
+    # batch) and in a batch of two
     say(f"radix bits {bits}, sort tile {tile}, raster mode {mode}, batch {batch}, longest first {longest}")
     case = Case(Workload("clustered", 300_000, seed=5),
                 config(radix_bits_per_digit=bits, sort_tile_keys=tile, raster_mode=mode, raster_batch=batch,
-                       raster_longest_first=longest), 800, 600, sphere_pose(3))
-    check_case(case, conics=False)
+                       raster_longest_first=longest, max_views=2), 800, 600, sphere_pose(3))
+    img = check_case(case, conics=False)
+    entries = case.renderer.read_entries()
+    assert sa.sort_tiles(case.cfg, 300_000, 2) == (tile, tile)
+    other = sa.Frame(device(), 320, 240)
+    case.renderer.render_views([other, case.frame], [case.cam] * 2, [case.view] * 2, case.scene)
+    for view in (0, 1):  # the visible set and order do not depend on the frame's size (same aspect)
+        case.renderer.select_view(view)
+        assert all(np.array_equal(a, b) for a, b in zip(case.renderer.read_entries(), entries))
+    assert np.array_equal(case.frame.read()[..., [2, 1, 0, 3]], img)
 
 
 @pytest.mark.parametrize("mode,unaligned,blend", [(0, True, sa.BlendMode.F32), (0, False, sa.BlendMode.UNORM8),
@@ -165,14 +175,13 @@ def test_wide_frame_uses_pixel_boxes():
     check_case(case, conics=False)
 
 
-@pytest.mark.parametrize("scale,search", [(1.0, False), (12.0, True)])
-def test_bin_owner_table_and_search(scale, search):
-    """The binning expands a block's 1024 entries (in depth order) through an
-    owner table when they emit at most 4096 pairs, and by binary search over
-    their offsets when they emit more.  More pairs than 4096 per block of
-    the frame put at least one block above 4096; fewer than four per splat
-    put at least one at or below it.  Either way the frame equals the
-    oracle's."""
+@pytest.mark.parametrize("scale,rounds", [(1.0, False), (12.0, True)])
+def test_bin_owner_table_in_one_round_and_in_several(scale, rounds):
+    """The binning expands a tile's 256 entries (in depth order) through an
+    owner table, 4096 output slots at a time.  More pairs than 4096 for every
+    tile of the frame put at least one tile's above 4096, in several rounds;
+    fewer than four per splat are at most a thousand a tile on average, so at
+    least one takes one round.  Either way the frame equals the oracle's."""
     say(f"splat scale {scale}")
     case = Case(Workload("gaussian", 60_000, seed=21), config(splat_scale=scale), 640, 480,
                 sphere_pose(21, radius=4))
@@ -180,8 +189,8 @@ def test_bin_owner_table_and_search(scale, search):
     pairs, visible = case.renderer.pair_count(), case.renderer.visible_count()
     say(f"  pairs {pairs}, visible {visible}, {pairs / max(visible, 1):.2f} a splat")
     assert visible > 4096
-    blocks = -(-visible // 1024)
-    assert (pairs > 4096 * blocks) if search else (pairs < 4 * visible)
+    tiles = -(-visible // 256)
+    assert (pairs > 4096 * tiles) if rounds else (pairs < 4 * visible)
 
 
 def test_edge_cases_empty_culled_tiny_ragged():
@@ -242,6 +251,67 @@ def test_malformed_records():
     d = image_diff(img, oimg)
     say(f"  image max diff {d}/255")
     assert d <= IMAGE_TOL and (img[..., 3] < 255).mean() > 0.2
+
+
+def malformed(rec, cam):
+    """The records of test_malformed_records, in twelfths of `rec`."""
+    rec = rec.copy()
+    part = [slice(k, None, 12) for k in range(12)]
+    rec["rotation"][part[0]] = 0.0
+    rec["center"][part[1]] = np.nan
+    rec["scale"][part[2]] = -np.inf
+    rec["scale"][part[3]] = 1e3
+    rec["alpha"][part[4]] = 1e30
+    rec["alpha"][part[5]] = -1e30
+    rec["color"][part[6]] = np.nan
+    rec["color"][part[7]] = 1e30
+    rec["center"][part[8]] = cam[3, :3]
+    rec["scale"][part[9], 0] = -30.0
+    rec["rotation"][part[10]] = np.inf
+    return rec
+
+
+# Malformed records in the forms that test_malformed_records does not reach:
+# in a list that has blocks of its own (3000 faint splats, all in the one tile of
+# a 16x16 frame), and in every walk of ordinary tiles (lists below 512).
+@pytest.mark.parametrize("unaligned,blend", [(True, sa.BlendMode.UNORM8), (False, sa.BlendMode.UNORM8),
+                                             (True, sa.BlendMode.F32), (False, sa.BlendMode.F32)])
+@pytest.mark.parametrize("heavy,mode", [(True, 3), (False, 0), (False, 1), (False, 2), (False, 3)])
+def test_malformed_records_in_every_walk(heavy, mode, unaligned, blend):
+    say(f"malformed records, heavy list {heavy}, mode {mode}, unaligned {unaligned}, blend {blend}")
+    n, (width, height) = (3000, (16, 16)) if heavy else (6000, (480, 360))
+    cam, view = sphere_pose(22, radius=5)
+    case = Case(Workload("gaussian", 0, seed=0),
+                config(raster_mode=mode, use_unaligned_rectangles=unaligned, blend_mode=blend, max_splat_count=n,
+                       max_views=2, tile_pairs_per_splat=64), width, height, (cam, view))
+    rec = Workload("gaussian", n, seed=22).all()
+    if heavy:
+        rec["center"] *= 0.1
+        rec["scale"] += 2.0
+        rec["alpha"] = -4.0
+    rec = malformed(rec, cam)
+    case.records, case.splats = rec, ob.decode(rec)
+    case.scene = sa.Scene(case.renderer, n)
+    case.scene.load_records(0, rec)
+    case.renderer.enable_tile_stats(True)
+    img = case.render()
+    lens = case.renderer.tile_stats()[:, 0]
+    _, idx = case.renderer.read_entries()
+    _, oidx, orec, oimg = case.oracle()
+    assert np.array_equal(idx, oidx)
+    assert (~np.isfinite(orec)).any(axis=1).sum() > n // 12
+    assert lens[0] >= 512 if heavy else lens.max() < 512
+    d = image_diff(img, oimg)
+    say(f"  longest list {lens.max()}, image max diff {d}/255")
+    assert d <= IMAGE_TOL
+    # and in a batch of two, 256 entries a round
+    cfg = case.cfg
+    cfg.raster_batch = 256
+    r = sa.Renderer(device(), cfg)
+    frames = [sa.Frame(device(), width, height) for _ in range(2)]
+    r.render_views(frames, [cam] * 2, [view] * 2, case.scene)
+    got = frames[1].read()
+    assert np.array_equal(got[..., [2, 1, 0, 3]] if cfg.frame_format == sa.FrameFormat.BGRA8_UNORM else got, img)
 
 
 def test_deterministic_and_frame_size_changes():
