@@ -431,9 +431,9 @@ void launch_heavy_tiles(const HeavyLaunch& a, hipStream_t s) {
 // (ballot + mbcnt) and blends those; a wave whose 64 pixels are all opaque
 // stops blending, and the block stops when all four have.
 template <bool UNALIGNED, bool F32, int MODE, int B>
-// (mode 3 occupancy: 128-entry batches at seven waves per SIMD, 72 VGPRs,
-// one to three registers spilled outside the loops; the f32 blend needs
-// more and keeps six; 256-entry batches fit six at 84)
+// (mode 3 occupancy: 128-entry batches at seven waves per SIMD, 72 VGPRs, none
+// spilled; the f32 blend needs 78 or 79 and keeps six; 256-entry batches need
+// 84 to 86, and 31 KB of LDS, and run five)
 __global__ __launch_bounds__(256, MODE == 3 ? (B == 128 ? (F32 ? 6 : 7) : 5) : 1) void k_raster(RasterLaunch a) {
   static_assert(B == 128 || B == 256, "entries staged per batch");
   constexpr int U = B / 64;  // list slots per step of the entry-major walks

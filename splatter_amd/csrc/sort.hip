@@ -287,7 +287,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
   take_tiles(Int<ITEMS>{});
 }
 
-// Lanes and keys a lane of each tile size.  Few keys in all (`few`): eight or
+// Lanes and keys a lane of each tile size (renderer.cpp's sort_form has the
+// choice of tiles).  Few keys in all (`few`): eight or
 // four keys a lane shorten a tile's chain of rankings; one view, depth sort /
 // pair sort in us: 1M splats in 4096-key tiles of 512 x 8 lanes 55 / 39, of
 // 256 x 16 66 / 43; in 8192-key tiles of 1024 x 8 58 / 36, of 512 x 16

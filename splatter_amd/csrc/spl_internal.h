@@ -57,7 +57,8 @@ enum CounterSlot : int {
 };
 
 // Heavy tiles: lists of at least kHeavyMin pairs and 1 / kHeavyShare of the
-// batch's pairs (so never more than kHeavyCap of them).  An ordinary block
+// batch's pairs, rounded down, so kHeavyCap of them but for rounding (1001 lists
+// of 512 pairs): one past the cap stays an ordinary tile.  An ordinary block
 // takes about 11 ns for each entry of its list, the device about 25 entries a
 // ns over all tiles: a list of 1/275 of the pairs lasts as long as the whole
 // raster.  The share is some four times that, because a frame saturates most
