@@ -35,6 +35,9 @@ METRIC = "6M-splat 1080p frames/s batched vs plain; sort Gkeys/s; p50/p99 render
 HBM_PEAK_GBS = 8000.0
 # VALU issue peak: 256 CUs x 4 SIMDs x 2.4 GHz, one wave64 instruction per SIMD every 4 cycles
 VALU_PEAK_PER_S = 256 * 4 * 2.4e9 / 4
+# batches that a counter run of `--profile --steps 2 --warmup 1` launches: one
+# warm-up, two timed, the same two with stage events
+COUNTED_BATCHES = (0, 0, 1, 0, 1)
 STAGES = ["cull_key_compact", "digit_histograms", "depth_sort", "project", "bin", "pair_sort",
           "tile_ranges", "raster"]
 
@@ -487,6 +490,13 @@ def main() -> int:
         batch(k, [t_r])
     stage_ms = t_r.stage_times()
     t_r.enable_timing(False)
+    if not args.profile:
+        # and of the batches whose instructions the counter runs counted
+        t_r.enable_timing(True)
+        for k in COUNTED_BATCHES:
+            batch(k, [t_r])
+        counted_ms = t_r.stage_times()
+        t_r.enable_timing(False)
 
     if args.profile:
         copy_calibration()
@@ -555,16 +565,18 @@ def main() -> int:
     dom_name = STAGES[dom]
     launches = {"depth_sort": P, "pair_sort": Q}.get(dom_name, 1)
     achieved = nbytes[dom_name] / (stage_ms[dom] * 1e-3) / 1e9
-    # the raster is bound by VALU issue rather than HBM: its wave instructions
-    # per launch (counters of the same workload) over the live launch time
+    # the raster's traffic is far from the HBM's rate: its wave instructions per
+    # launch (counters of the same workload) over the live time of the same
+    # batches, a mark and not a proven limit
     valu = measured_valu(dom_name)
     valu_issue = None
     if valu and launches == 1:
-        rate = valu[1] / (stage_ms[dom] * 1e-3 * V_PER)
+        rate = valu[1] / (counted_ms[dom] * 1e-3 * V_PER)
         valu_issue = {"kernel": valu[0], "instructions_per_launch": valu[1], "achieved": round(rate / 1e9, 1),
                       "peak": round(VALU_PEAK_PER_S / 1e9, 1), "unit": "G wave64 VALU instructions/s",
                       "frac": round(rate / VALU_PEAK_PER_S, 4),
-                      "source": "SQ_INSTS_VALU per launch in profiles/kernels_6M_clustered_1080p_16views.md"}
+                      "source": "SQ_INSTS_VALU per launch in profiles/kernels_6M_clustered_1080p_16views.md, over "
+                                "the time of the batches counted there"}
     sort_i = STAGES.index("depth_sort")
     sort_gkeys = V / (stage_ms[sort_i] * 1e-3) / 1e9 if stage_ms[sort_i] > 0 else None
 
